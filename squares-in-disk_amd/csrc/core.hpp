@@ -69,6 +69,14 @@ struct DeviceCounters {
 };
 
 // A list of boxes in structure-of-arrays layout: lb[a * stride + i].
+//
+// A list that one level hands to the next may be kept in segments: segment g
+// holds the entries [g * seg_cap, g * seg_cap + count[g * kSegStride]).  Every
+// wave of the producing level appends its survivors with an atomic on a counter,
+// and atomics on one address from all XCDs serialise at about 12 ns each: with
+// one counter, the 51 K waves of Four's level 1 (3.3 M children) spent 610 of its
+// 663 us there.  The segments' counters lie in lines of their own (256 bytes
+// apart), and successive waves of children go to successive segments.
 struct BoxList {
     double* lb;
     double* ub;
@@ -77,8 +85,12 @@ struct BoxList {
     unsigned* leaf;      // static levels: enumeration index within that cuboid's grid
     unsigned long long stride;
     unsigned long long cap;
-    unsigned long long* count;  // device counter of valid entries
+    unsigned long long* count;  // device counter of valid entries (of each segment)
+    unsigned long long seg_cap; // entries of one segment (unsegmented: cap)
+    unsigned segs;              // segments: 1 or kSegs
 };
+constexpr unsigned kSegs = 16;
+constexpr unsigned kSegStride = 32;   // 64-bit words from one segment's counter to the next
 
 // Arguments of a level kernel.  The input range lives in device memory (the
 // round's pop position and size, or a list's counter), so a whole round can be
@@ -363,14 +375,89 @@ __device__ __forceinline__ unsigned long long wave_uniform(unsigned long long v)
     const unsigned hi = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(v >> 32));
     return (static_cast<unsigned long long>(hi) << 32) | lo;
 }
-__device__ __forceinline__ unsigned long long input_base(const LevelArgs& a) { return a.in_base ? *a.in_base : 0ull; }
-// Inputs [base, base + n) of a level, n clamped to the input list's capacity (a
-// count past it was raised by a pass that could not store its survivors, which
-// set the overflow flag and fails the call).
-__device__ __forceinline__ unsigned long long input_count(const LevelArgs& a, unsigned long long base) {
+// The inputs of a level: n of them, numbered segment by segment where the list is
+// segmented.  Counts are clamped to the list's (or segment's) capacity (a count
+// past it was raised by a pass that could not store its survivors, which set the
+// overflow flag and fails the call).
+//
+// One wave of the block reads and sums the segments' counters (16 lines; done
+// by every wave, and 32 of them, it cost batched prefiltered One 6%), every wave
+// keeps the sums in its lanes (lane g: the inputs before segment g) and finds the
+// segment of its first input with one ballot (a search per lane in LDS: 20%).
+// SEG = false: the level's input list is dense (the first level of its kind).
+template<bool SEG>
+struct Inputs {
+    bool dense;
+    unsigned before;                    // segmented lists hold less than 2^32 entries
+    unsigned long long base, n, seg_cap;
+    // The list entry of input `item`, for items that do not decrease over the
+    // lanes; called by every lane of the wave (`valid` marks those that need it).
+    __device__ __forceinline__ unsigned long long entry(unsigned long long item64, bool valid) const {
+        if(!SEG || dense) return base + item64;
+        const unsigned item = static_cast<unsigned>(item64);
+        const unsigned first = __builtin_amdgcn_readfirstlane(item);
+        unsigned g = static_cast<unsigned>(__popcll(__ballot(before <= first) & ((1ull << kSegs) - 1ull))) - 1u;
+        unsigned from = __builtin_amdgcn_readlane(before, g), to = __builtin_amdgcn_readlane(before, g + 1u);
+        unsigned long long at = g * seg_cap + (item - from);
+        bool beyond = valid && item >= to;
+        while(__ballot(beyond)) {
+            ++g;
+            from = to;
+            to = __builtin_amdgcn_readlane(before, g + 1u);
+            if(beyond) {
+                at = g * seg_cap + (item - from);
+                beyond = item >= to;
+            }
+        }
+        return at;
+    }
+};
+// v plus the value SHIFT lanes below (0 past the row's first lane) in rows of 16 lanes.
+template<int SHIFT> __device__ __forceinline__ unsigned row_add(unsigned v) {
+    return v + static_cast<unsigned>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x110 + SHIFT, 0xf, 0xf, false));
+}
+// Called by every thread of the block.
+template<bool SEG>
+__device__ __forceinline__ Inputs<SEG> level_inputs(const LevelArgs& a) {
+    Inputs<SEG> in;
+    in.seg_cap = a.in.seg_cap;
+    in.base = a.in_base ? *a.in_base : 0ull;
+    in.dense = true;
+    in.before = 0;
+    if constexpr(SEG) {
+        static_assert(kSegs == 16, "the scan covers one row of 16 lanes");
+        in.dense = a.in.segs <= 1;
+        if(!in.dense) {
+            __shared__ unsigned s_before[64];
+            if(threadIdx.x < 64) {
+                unsigned v = 0;
+                if(threadIdx.x < kSegs) {
+                    const unsigned long long n = a.in_count[threadIdx.x * kSegStride];
+                    v = static_cast<unsigned>(n < a.in.seg_cap ? n : a.in.seg_cap);
+                }
+                const unsigned sum = row_add<8>(row_add<4>(row_add<2>(row_add<1>(v))));
+                s_before[threadIdx.x] = threadIdx.x < kSegs ? sum - v : __builtin_amdgcn_readlane(sum, kSegs - 1);
+            }
+            __syncthreads();
+            in.before = s_before[__lane_id()];
+            in.n = __builtin_amdgcn_readlane(in.before, kSegs);
+            return in;
+        }
+    }
     const unsigned long long n = *a.in_count;
-    const unsigned long long room = a.in.cap > base ? a.in.cap - base : 0ull;
-    return n < room ? n : room;
+    const unsigned long long room = a.in.cap > in.base ? a.in.cap - in.base : 0ull;
+    in.n = n < room ? n : room;
+    return in;
+}
+// Appends the flagged lanes to segment `seg` (any number, taken modulo the
+// list's segments; the same on all lanes): the entry's place, or ~0 when the
+// segment is full.  SEG = false: the list is dense (the last level of its kind).
+// Called by every lane of the wave.
+template<bool SEG>
+__device__ __forceinline__ unsigned long long list_append(const BoxList& l, bool flag, unsigned seg) {
+    const unsigned s = !SEG || l.segs <= 1 ? 0u : seg % kSegs;
+    const unsigned long long pos = wave_append(flag, l.count + static_cast<unsigned long long>(s) * kSegStride);
+    return pos < l.seg_cap ? s * l.seg_cap + pos : ~0ull;
 }
 
 template<class P>
@@ -474,20 +561,20 @@ __device__ __forceinline__ int group_size(const LevelArgs& args, unsigned long l
     return 1;
 }
 
-// Child w of a static level: the parent box with the level's variable replaced
-// by subrange w % SUBS of the splitter (splitter.hpp:44-59), its dynamic cuboid
-// (origin) and its enumeration index within that cuboid's grid (leaf).
+// Child w of a static level, counted over the entries of its input list: the
+// parent box at entry w / SUBS with the level's variable replaced by subrange
+// w % SUBS of the splitter (splitter.hpp:44-59), its dynamic cuboid (origin) and
+// its enumeration index within that cuboid's grid (leaf).
 template<class P, int L>
-__device__ __forceinline__ void static_child(const LevelArgs& args, unsigned long long in_base, unsigned long long w,
+__device__ __forceinline__ void static_child(const LevelArgs& args, const Inputs<(L > 0)>& in, unsigned long long w,
                                              double (&lb)[P::N], double (&ub)[P::N], unsigned& origin, unsigned& leaf) {
     constexpr int ARG = P::st_arg(L);
     constexpr int SUBS = P::st_subs(L);
-    const unsigned long long item = w / SUBS;
+    const unsigned long long src = w / SUBS;
     const int i = static_cast<int>(w % SUBS);
-    const unsigned long long src = in_base + item;
     load_box<P>(args.in, src, lb, ub);
     if(args.in.origin) { origin = args.in.origin[src]; leaf = args.in.leaf[src]; }
-    else { origin = static_cast<unsigned>(item); leaf = 0; }
+    else { origin = static_cast<unsigned>(src - in.base); leaf = 0; }
     leaf = leaf * SUBS + static_cast<unsigned>(i);
     const double pl = lb[ARG], pu = ub[ARG];
     const double wd = split_width(pl, pu, SUBS);
@@ -499,10 +586,11 @@ __device__ __forceinline__ void static_child(const LevelArgs& args, unsigned lon
 // check the level's constraint rows, then count the leaf, join the hull (last
 // non-final level), record a critical (last final level) or append the survivor
 // to the next level's list.  Called by every lane of the wave (the hull join and
-// the append are wave-wide); `valid` marks the lanes that hold a child.
+// the append are wave-wide); `valid` marks the lanes that hold a child, `seg` is
+// the output segment of the wave's survivors.
 template<class P, int MODE, int L>
-__device__ __forceinline__ void static_decide(const LevelArgs& args, unsigned long long in_base, bool valid,
-                                              unsigned long long w, const double* s_c, PropScratch<P>& s_prop,
+__device__ __forceinline__ void static_decide(const LevelArgs& args, const Inputs<(L > 0)>& in, bool valid,
+                                              unsigned long long w, unsigned seg, const double* s_c, PropScratch<P>& s_prop,
                                               unsigned long long& c_leaf, unsigned long long& c_crit) {
     constexpr int N = P::N;
     constexpr int ARG = P::st_arg(L);
@@ -511,7 +599,7 @@ __device__ __forceinline__ void static_decide(const LevelArgs& args, unsigned lo
     double lb[N], ub[N];
     unsigned origin = 0, leaf = 0;
     if(valid) {
-        static_child<P, L>(args, in_base, w, lb, ub, origin, leaf);
+        static_child<P, L>(args, in, w, lb, ub, origin, leaf);
         if(propagate<P, P::prop_fast(L)>(lb, ub, ARG, N, 4u, s_c, s_prop)) {
             ++c_leaf;
         } else if(P::template rows_violated<L>(lb, ub, s_c)) {
@@ -526,9 +614,9 @@ __device__ __forceinline__ void static_decide(const LevelArgs& args, unsigned lo
     }
     if(LAST && MODE == NONFINAL) hull_join<N>(args.hull, join, origin, leaf, lb, ub);
     if(!LAST || MODE == FINAL) {
-        const unsigned long long pos = wave_append(survive, args.out.count);
+        const unsigned long long pos = list_append<!LAST>(args.out, survive, seg);
         if(survive) {
-            if(pos < args.out.cap) {
+            if(pos != ~0ull) {
                 store_box<P>(args.out, pos, lb, ub);
                 if(args.out.origin) { args.out.origin[pos] = origin; args.out.leaf[pos] = leaf; }
             } else if(!LAST) {
@@ -556,7 +644,7 @@ __device__ __forceinline__ void static_decide_hoisted(const LevelArgs& args, boo
                                                       const double (&pub)[P::N], double pl, double pu, double wd, int i,
                                                       unsigned origin, unsigned leaf,
                                                       const typename P::template Hoist<L, double>& h,
-                                                      const double* s_c, PropScratch<P>& s_prop,
+                                                      unsigned seg, const double* s_c, PropScratch<P>& s_prop,
                                                       unsigned long long& c_leaf, unsigned long long& c_crit,
                                                       bool& defer) {
     constexpr int N = P::N;
@@ -603,9 +691,9 @@ __device__ __forceinline__ void static_decide_hoisted(const LevelArgs& args, boo
     }
     if(LAST && MODE == NONFINAL) hull_join<N>(args.hull, join, origin, leaf, lb, ub);
     if(!LAST || MODE == FINAL) {
-        const unsigned long long pos = wave_append(survive, args.out.count);
+        const unsigned long long pos = list_append<!LAST>(args.out, survive, seg);
         if(survive) {
-            if(pos < args.out.cap) {
+            if(pos != ~0ull) {
                 store_box<P>(args.out, pos, lb, ub);
                 if(args.out.origin) { args.out.origin[pos] = origin; args.out.leaf[pos] = leaf; }
             } else if(!LAST) {
@@ -642,8 +730,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(static_l
 void k_static_level(LevelArgs job0) {
     const LevelArgs args = job_args(job0);
     constexpr int SUBS = P::st_subs(L);
-    const unsigned long long in_base = input_base(args);
-    const unsigned long long n_items = input_count(args, in_base);
+    const Inputs<(L > 0)> in = level_inputs<(L > 0)>(args);
+    const unsigned long long n_items = in.n;
     // the list holds at most undec_cap entries; a pass that found more counted
     // them (and raised the overflow flag, which fails the call) but stored only
     // those that fit
@@ -681,7 +769,7 @@ void k_static_level(LevelArgs job0) {
         // and decided 64 at a time, so that a wave does not run that path for
         // one or two of its lanes.  The list holds fewer than 64 children
         // between parents, so 64 + SUBS entries suffice.
-        constexpr bool DEFER = P::prop_fast(L);
+        constexpr bool DEFER = P::prop_fast(L) && L == P::NSTAT - 1;
         __shared__ unsigned long long s_def[kBlock / 64][DEFER ? 64 + SUBS : 1];
         unsigned long long* const dq = s_def[wib];
         unsigned dcount = 0;   // wave-uniform
@@ -690,18 +778,17 @@ void k_static_level(LevelArgs job0) {
         const unsigned long long waves = static_cast<unsigned long long>(gridDim.x) * (blockDim.x / 64);
         const unsigned long long wave = static_cast<unsigned long long>(blockIdx.x) * (blockDim.x / 64) + wib;
         const unsigned long long items = wave_uniform(n_items);
-        const unsigned long long base = wave_uniform(in_base);
         const unsigned long long wtrips = (items + waves - 1) / waves;   // the same for every wave
         for(unsigned long long trip = 0; trip < wtrips; ++trip) {
             const unsigned long long item = wave + trip * waves;
             const bool valid = item < items;                              // wave-uniform
+            const unsigned long long src = wave_uniform(in.entry(item, valid));
             double plb[N], pub[N];
             double pl = 0, pu = 0, wd = 0;
             unsigned p_origin = 0, p_leaf = 0;
 #pragma unroll
             for(int a = 0; a < N; ++a) { plb[a] = 0.0; pub[a] = 0.0; }
             if(valid) {
-                const unsigned long long src = base + item;
                 load_box<P>(args.in, src, plb, pub);
                 if(args.in.origin) { p_origin = args.in.origin[src]; p_leaf = args.in.leaf[src]; }
                 else { p_origin = static_cast<unsigned>(item); p_leaf = 0; }
@@ -719,11 +806,12 @@ void k_static_level(LevelArgs job0) {
                 const int i = lane + 64 * k;
                 bool defer;
                 static_decide_hoisted<P, MODE, L, DEFER>(args, valid, plb, pub, pl, pu, wd, i, p_origin,
-                                                         p_leaf * SUBS + static_cast<unsigned>(i), h, s_c, s_prop,
+                                                         p_leaf * SUBS + static_cast<unsigned>(i), h,
+                                                         static_cast<unsigned>(item) * (SUBS / 64) + k, s_c, s_prop,
                                                          c_leaf, c_crit, defer);
                 if constexpr(DEFER) {
                     const unsigned long long m = __ballot(defer);
-                    if(defer) dq[dcount + __popcll(m & below)] = item * SUBS + static_cast<unsigned>(i);
+                    if(defer) dq[dcount + __popcll(m & below)] = src * SUBS + static_cast<unsigned>(i);
                     dcount += static_cast<unsigned>(__popcll(m));
                 }
             }
@@ -738,7 +826,7 @@ void k_static_level(LevelArgs job0) {
                     dcount -= take;
                     const bool v = static_cast<unsigned>(lane) < take;
                     const unsigned long long w = v ? dq[dcount + lane] : 0ull;
-                    static_decide<P, MODE, L>(args, base, v, w, s_c, s_prop, c_leaf, c_crit);
+                    static_decide<P, MODE, L>(args, in, v, w, 0u, s_c, s_prop, c_leaf, c_crit);
                 }
                 __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
                 __builtin_amdgcn_wave_barrier();
@@ -749,10 +837,17 @@ void k_static_level(LevelArgs job0) {
         for(unsigned long long trip = 0; trip < trips; ++trip) {
             const unsigned long long t = first + trip * stride;
             const bool valid = t < total;
-            unsigned long long w = t;
-            if(F32) w = valid ? args.undec[t] : 0ull;
-            else if(valid && w % SUBS == 0) c_cub += SUBS;
-            static_decide<P, MODE, L>(args, in_base, valid, w, s_c, s_prop, c_leaf, c_crit);
+            unsigned long long w = 0;
+            if(F32) {
+                if(valid) w = args.undec[t];
+            } else {
+                w = in.entry(t / SUBS, valid) * SUBS + t % SUBS;
+                if(valid && t % SUBS == 0) c_cub += SUBS;
+            }
+            // successive waves of children append to successive segments, so a
+            // segment receives at most its share of them and one wave more
+            const unsigned seg = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(t / 64));
+            static_decide<P, MODE, L>(args, in, valid, w, seg, s_c, s_prop, c_leaf, c_crit);
         }
     }
     block_counts_add(args.block_counts, c_cub, c_leaf, MODE == FINAL ? c_crit : 0ull);
@@ -797,8 +892,8 @@ __global__ __launch_bounds__(kBlock) SQD_LEVEL_ATTR void k_static_prefilter(Leve
     const float* const s_c32 = nullptr;
     __shared__ PropScratch<P> s_prop;
     enter_round_down();
-    const unsigned long long in_base = input_base(args);
-    const unsigned long long n_items = input_count(args, in_base);
+    const Inputs<(L > 0)> in = level_inputs<(L > 0)>(args);
+    const unsigned long long n_items = in.n;
     const unsigned long long stride = static_cast<unsigned long long>(gridDim.x) * blockDim.x;
     const int cpl = group_size<SUBS, CPL>(args, n_items, stride);
     const int step = SUBS / cpl;                                                       // groups per parent
@@ -806,7 +901,8 @@ __global__ __launch_bounds__(kBlock) SQD_LEVEL_ATTR void k_static_prefilter(Leve
     const unsigned long long first = static_cast<unsigned long long>(blockIdx.x) * blockDim.x + threadIdx.x;
     if(static_cast<unsigned long long>(blockIdx.x) * blockDim.x >= total) return;   // no groups in any trip (block-uniform)
     const unsigned long long trips = (total + stride - 1) / stride;
-    __shared__ unsigned long long s_groups[kBlock];   // the trip's groups that the group test left
+    // the trip's groups that the group test left, and the entries of their parents
+    __shared__ unsigned long long s_groups[kBlock], s_entry[kBlock];
     __shared__ unsigned long long s_ngroups;
     // The hoisted terms of the parents of one block trip (at most MAXP of them:
     // a trip's kBlock consecutive groups, at least SUBS / CPL per parent), kept
@@ -825,6 +921,7 @@ __global__ __launch_bounds__(kBlock) SQD_LEVEL_ATTR void k_static_prefilter(Leve
         const unsigned long long s0 = static_cast<unsigned long long>(blockIdx.x) * blockDim.x + trip * stride;
         const unsigned long long item0 = s0 / static_cast<unsigned long long>(step);   // the trip's first parent
         const unsigned long long slot = first + trip * stride;
+        const unsigned long long src = in.entry(slot / static_cast<unsigned long long>(step), slot < total);
         bool keep = false;
         if(slot < total) {
             const unsigned long long item = slot / static_cast<unsigned long long>(step);
@@ -833,7 +930,7 @@ __global__ __launch_bounds__(kBlock) SQD_LEVEL_ATTR void k_static_prefilter(Leve
             keep = true;
             if(cpl > 1 || SHARE) {
                 double lb[N], ub[N];
-                load_box<P>(args.in, in_base + item, lb, ub);
+                load_box<P>(args.in, src, lb, ub);
                 float hl[N], hu[N];
 #pragma unroll
                 for(int a = 0; a < N; ++a) { hl[a] = f32_down(lb[a]); hu[a] = f32_up(ub[a]); }
@@ -856,7 +953,10 @@ __global__ __launch_bounds__(kBlock) SQD_LEVEL_ATTR void k_static_prefilter(Leve
             }
         }
         const unsigned long long at = wave_append(keep, &s_ngroups);
-        if(keep) s_groups[at] = slot;
+        if(keep) {
+            s_groups[at] = slot;
+            s_entry[at] = src;
+        }
         __syncthreads();
         // 2. the children of the groups left, spread over the block's lanes
         const unsigned long long m = s_ngroups * static_cast<unsigned long long>(cpl);
@@ -866,12 +966,13 @@ __global__ __launch_bounds__(kBlock) SQD_LEVEL_ATTR void k_static_prefilter(Leve
             unsigned long long w = 0;
             if(q < m) {
                 const unsigned long long gs = s_groups[q / static_cast<unsigned long long>(cpl)];
+                const unsigned long long src = s_entry[q / static_cast<unsigned long long>(cpl)];
                 const unsigned long long item = gs / static_cast<unsigned long long>(step);
                 const int i = static_cast<int>(gs % static_cast<unsigned long long>(step)) * cpl +
                               static_cast<int>(q % static_cast<unsigned long long>(cpl));
-                w = item * SUBS + static_cast<unsigned long long>(i);
+                w = src * SUBS + static_cast<unsigned long long>(i);
                 double lb[N], ub[N];
-                load_box<P>(args.in, in_base + item, lb, ub);
+                load_box<P>(args.in, src, lb, ub);
                 float plb[N], pub[N];
 #pragma unroll
                 for(int a = 0; a < N; ++a) { plb[a] = f32_down(lb[a]); pub[a] = f32_up(ub[a]); }
@@ -935,8 +1036,8 @@ __global__ __launch_bounds__(kBlock) SQD_LEVEL_ATTR void k_static_group64(LevelA
     constexpr int CPL = children_per_lane<SUBS>();
     const double* const s_c = nullptr;   // constants are literals in the generated code (P::kc)
     enter_round_down();
-    const unsigned long long in_base = input_base(args);
-    const unsigned long long n_items = input_count(args, in_base);
+    const Inputs<(L > 0)> in = level_inputs<(L > 0)>(args);
+    const unsigned long long n_items = in.n;
     const unsigned long long stride = static_cast<unsigned long long>(gridDim.x) * blockDim.x;
     const int cpl = group_size<SUBS, CPL>(args, n_items, stride);
     const int step = SUBS / cpl;                                                       // groups per parent
@@ -947,17 +1048,17 @@ __global__ __launch_bounds__(kBlock) SQD_LEVEL_ATTR void k_static_group64(LevelA
     unsigned long long c_cub = 0, c_leaf = 0;
     for(unsigned long long trip = 0; trip < trips; ++trip) {
         const unsigned long long slot = first + trip * stride;
+        const unsigned long long src = in.entry(slot / static_cast<unsigned long long>(step), slot < total);
         bool keep = false;
         unsigned long long w0 = 0;
         if(slot < total) {
-            const unsigned long long item = slot / static_cast<unsigned long long>(step);
             const int g = static_cast<int>(slot % static_cast<unsigned long long>(step));
             if(g == 0) c_cub += SUBS;
-            w0 = item * SUBS + static_cast<unsigned long long>(g * cpl);
+            w0 = src * SUBS + static_cast<unsigned long long>(g * cpl);
             keep = true;
             if(cpl > 1) {
                 double lb[N], ub[N];
-                load_box<P>(args.in, in_base + item, lb, ub);
+                load_box<P>(args.in, src, lb, ub);
                 typename P::template Hoist<L, double> h;
                 P::template hoist<L>(lb, ub, s_c, h);
                 const double pl = lb[ARG], pu = ub[ARG];
@@ -997,8 +1098,8 @@ __global__ __launch_bounds__(kBlock) SQD_LEVEL_ATTR void k_dynamic_level(LevelAr
     const double* const s_c = nullptr;   // constants are literals in the generated code (P::kc)
     __shared__ PropScratch<P> s_prop;
     enter_round_down();
-    const unsigned long long in_base = input_base(args);
-    const unsigned long long n_items = input_count(args, in_base);
+    const Inputs<(J > 0)> in = level_inputs<(J > 0)>(args);
+    const unsigned long long n_items = in.n;
     // the initial queue may start from a range of the first variable's subdivisions
     constexpr bool RANGED = (MODE == INIT && J == 0);
     const unsigned long long r_lo = RANGED && args.init_range ? args.init_range[0] : 0ull;
@@ -1014,10 +1115,9 @@ __global__ __launch_bounds__(kBlock) SQD_LEVEL_ATTR void k_dynamic_level(LevelAr
         bool survive = false;
         double lb[N], ub[N];
         unsigned depth = 0;
+        const unsigned long long src = in.entry(w / r_n, w < total);
         if(w < total) {
-            const unsigned long long item = w / r_n;
             const int i = static_cast<int>(r_lo + w % r_n);
-            const unsigned long long src = in_base + item;
             load_box<P>(args.in, src, lb, ub);
             depth = args.in.depth ? args.in.depth[src] : 0u;
             ++c_cub;
@@ -1033,9 +1133,10 @@ __global__ __launch_bounds__(kBlock) SQD_LEVEL_ATTR void k_dynamic_level(LevelAr
                 survive = true;
             }
         }
-        const unsigned long long pos = wave_append(survive, args.out.count);
+        const unsigned long long pos =
+            list_append<!LAST>(args.out, survive, __builtin_amdgcn_readfirstlane(static_cast<unsigned>(w / 64)));
         if(survive) {
-            if(pos < args.out.cap) {
+            if(pos != ~0ull) {
                 store_box<P>(args.out, pos, lb, ub);
                 if(args.out.depth) args.out.depth[pos] = depth;
             } else {

@@ -68,10 +68,20 @@ unsigned blocks_per_cu(K kernel) {
 }
 // Rows of a level launch: one per job of the batch (job_args).
 inline unsigned jobs_of(const dev::LevelArgs& a) { return a.jobs ? a.jobs : 1u; }
-inline unsigned level_grid(unsigned resident, unsigned long long max_children, unsigned grid) {
+// Blocks of one row of a level launch of `jobs` rows: the resident capacity up to
+// 8 rows, then the rows share 8 times that, down to one block per compute unit.  A
+// row's blocks beyond its work, and the rows without any (49 K blocks in a batch
+// of 32), still have to start, read their input's size and leave: an empty launch
+// of One's batches of 32 took 18 us, and the whole batch 403 us against 343 us at
+// 256 blocks per row.  A batch of few rows keeps the capacity per row, since one
+// job is often left alone in it: at 384 blocks per row the job stream in
+// batches of 4 took 14.6 ms instead of 11.3.
+inline unsigned level_grid(unsigned per_cu, unsigned cus, unsigned jobs, unsigned long long max_children, unsigned grid) {
     if(grid) return grid;
+    const unsigned share = jobs > 8 ? per_cu * cus * 8 / jobs : per_cu * cus;
+    const unsigned most = share > cus ? share : cus;
     const unsigned long long need = (max_children + dev::kBlock - 1) / dev::kBlock;
-    return static_cast<unsigned>(need < 1 ? 1 : (need < resident ? need : resident));
+    return static_cast<unsigned>(need < 1 ? 1 : (need < most ? need : most));
 }
 
 // One static level: the binary64 kernel over every child, or (F32) the binary32
@@ -81,14 +91,14 @@ hipError_t launch_one_static(const dev::LevelArgs& a, unsigned long long max_chi
                              hipStream_t s) {
     if(F32) {
         static const unsigned pre_cu = blocks_per_cu(dev::k_static_prefilter<P, MODE, L>);
-        hipLaunchKernelGGL((dev::k_static_prefilter<P, MODE, L>), dim3(level_grid(pre_cu * cus, max_children, grid), jobs_of(a)),
+        hipLaunchKernelGGL((dev::k_static_prefilter<P, MODE, L>), dim3(level_grid(pre_cu, cus, jobs_of(a), max_children, grid), jobs_of(a)),
                            dim3(dev::kBlock), 0, s, a);
         const hipError_t e = hipGetLastError();
         if(e != hipSuccess) return e;
     }
     static const unsigned per_cu = blocks_per_cu(dev::k_static_level<P, MODE, L, F32>);
     hipLaunchKernelGGL((dev::k_static_level<P, MODE, L, F32>),
-                       dim3(level_grid(per_cu * cus, max_children, grid), jobs_of(a)), dim3(dev::kBlock), 0, s, a);
+                       dim3(level_grid(per_cu, cus, jobs_of(a), max_children, grid), jobs_of(a)), dim3(dev::kBlock), 0, s, a);
     return hipGetLastError();
 }
 // One static level with the binary64 group test: the test, then the binary64
@@ -98,12 +108,12 @@ hipError_t launch_one_grouped(const dev::LevelArgs& a, unsigned long long max_ch
                               hipStream_t s) {
     static const unsigned pre_cu = blocks_per_cu(dev::k_static_group64<P, MODE, L>);
     hipLaunchKernelGGL((dev::k_static_group64<P, MODE, L>),
-                       dim3(level_grid(pre_cu * cus, max_children, grid), jobs_of(a)), dim3(dev::kBlock), 0, s, a);
+                       dim3(level_grid(pre_cu, cus, jobs_of(a), max_children, grid), jobs_of(a)), dim3(dev::kBlock), 0, s, a);
     const hipError_t e = hipGetLastError();
     if(e != hipSuccess) return e;
     static const unsigned per_cu = blocks_per_cu(dev::k_static_level<P, MODE, L, true>);
     hipLaunchKernelGGL((dev::k_static_level<P, MODE, L, true>),
-                       dim3(level_grid(per_cu * cus, max_children, grid), jobs_of(a)), dim3(dev::kBlock), 0, s, a);
+                       dim3(level_grid(per_cu, cus, jobs_of(a), max_children, grid), jobs_of(a)), dim3(dev::kBlock), 0, s, a);
     return hipGetLastError();
 }
 template<class P, int MODE, int... L>
@@ -119,7 +129,7 @@ hipError_t launch_one_dynamic(const dev::LevelArgs& a, unsigned long long max_ch
                               hipStream_t s) {
     static const unsigned per_cu = blocks_per_cu(dev::k_dynamic_level<P, MODE, J>);
     hipLaunchKernelGGL((dev::k_dynamic_level<P, MODE, J>),
-                       dim3(level_grid(per_cu * cus, max_children, grid), jobs_of(a)), dim3(dev::kBlock), 0, s, a);
+                       dim3(level_grid(per_cu, cus, jobs_of(a), max_children, grid), jobs_of(a)), dim3(dev::kBlock), 0, s, a);
     return hipGetLastError();
 }
 template<class P, int MODE, bool F32, int... L>

@@ -77,6 +77,19 @@ struct DeviceState {
 
 static_assert(sizeof(DeviceState) % sizeof(unsigned long long) == 0, "state is a block of 64-bit words");
 
+// The counters of a core's segmented level lists (dev::BoxList): n_lists blocks
+// of dev::kSegs counters, dev::kSegStride words apart (n_lists = 0: none).
+struct SegCounters {
+    unsigned long long* p;
+    unsigned n_lists;
+};
+// The job's segment counters to zero (by all threads of one block).
+__device__ __forceinline__ void segment_counters_reset(SegCounters s, unsigned long long job_off) {
+    unsigned long long* p = dev::job_ptr(s.p, job_off);
+    for(unsigned i = threadIdx.x; i < s.n_lists * dev::kSegs; i += blockDim.x)
+        p[static_cast<unsigned long long>(i) * dev::kSegStride] = 0ull;
+}
+
 __global__ void k_set_u64(unsigned long long* p, unsigned long long v) {
     if(threadIdx.x == 0 && blockIdx.x == 0) *p = v;
 }
@@ -90,7 +103,7 @@ __global__ void k_set_u64(unsigned long long* p, unsigned long long v) {
 __global__ void k_proof_start(unsigned long long* words, unsigned n_words, const double* box, int n_args,
                               double* list_lb, double* list_ub, unsigned* list_depth, unsigned long long list_stride,
                               unsigned long long count_word, const unsigned long long* start_flag,
-                              unsigned long long stride) {
+                              SegCounters segs, unsigned long long stride) {
     const unsigned long long off = dev::job_offset(stride);
     words = dev::job_ptr(words, off);
     box = dev::job_ptr(box, off);
@@ -108,6 +121,7 @@ __global__ void k_proof_start(unsigned long long* words, unsigned n_words, const
         list_lb[static_cast<unsigned long long>(a) * list_stride] = box[a];
         list_ub[static_cast<unsigned long long>(a) * list_stride] = box[n_args + a];
     }
+    segment_counters_reset(segs, off);
     if(threadIdx.x == 0 && list_depth) list_depth[0] = 0u;
     __syncthreads();
     if(threadIdx.x == 0) words[count_word] = 1ull;
@@ -135,8 +149,10 @@ __global__ void k_set_ranges(unsigned long long* p, unsigned long long stride, J
 }
 // Start of a proof (or of a host-driven call): the whole control block (state
 // and per-block count slots) to zero.
-__global__ void k_state_reset(unsigned long long* words, unsigned long long n_words, unsigned long long stride) {
+__global__ void k_state_reset(unsigned long long* words, unsigned long long n_words, SegCounters segs,
+                              unsigned long long stride) {
     words = dev::job_ptr(words, dev::job_offset(stride));
+    if(blockIdx.x == 0) segment_counters_reset(segs, dev::job_offset(stride));
     for(unsigned long long i = threadIdx.x; blockIdx.x == 0 && i < n_words; i += blockDim.x) words[i] = 0ull;
 }
 // The control blocks of a batch's jobs side by side in `out` (one copy to the host).
@@ -150,10 +166,11 @@ __global__ void k_gather_states(const unsigned long long* st, unsigned long long
 // the top of the stack (their slots are reused by the children the round
 // pushes), and clear the round's list counters.
 __global__ void k_round_begin(DeviceState* st, unsigned long long k_max, unsigned long long stack_cap,
-                              unsigned long long fanout, unsigned long long stride) {
+                              unsigned long long fanout, SegCounters segs, unsigned long long stride) {
     st = dev::job_ptr(st, dev::job_offset(stride));
     const unsigned t = threadIdx.x;
     if(blockIdx.x != 0) return;
+    segment_counters_reset(segs, dev::job_offset(stride));
     if(t == 0) {
         const unsigned long long S = st->stack_count;
         unsigned long long K = S < k_max ? S : k_max;
@@ -211,9 +228,23 @@ __global__ __launch_bounds__(kFoldThreads) void k_fold_counts(DeviceState* st, u
     }
 }
 // Level counters to zero (between chunks of a host-driven call).
-__global__ void k_levels_reset(DeviceState* st) {
+__global__ void k_levels_reset(DeviceState* st, SegCounters segs) {
+    if(blockIdx.x == 0) segment_counters_reset(segs, 0ull);
     if(blockIdx.x == 0 && threadIdx.x < 64) st->level_count[threadIdx.x] = 0;
     if(blockIdx.x == 0 && threadIdx.x < 32) st->undec_count[threadIdx.x] = 0;
+}
+// The totals of the segmented lists into the state's level counters, which the
+// host reads (profiling, final passes repeated in parts): list i is the output of
+// (mode, level) index[i].
+struct SegIndex { unsigned char index[64]; };
+__global__ void k_level_totals(DeviceState* st, SegCounters segs, SegIndex idx, unsigned long long stride) {
+    st = dev::job_ptr(st, dev::job_offset(stride));
+    const unsigned long long* p = dev::job_ptr(segs.p, dev::job_offset(stride));
+    for(unsigned i = threadIdx.x; i < segs.n_lists; i += blockDim.x) {
+        unsigned long long sum = 0;
+        for(unsigned g = 0; g < dev::kSegs; ++g) sum += p[static_cast<unsigned long long>(i * dev::kSegs + g) * dev::kSegStride];
+        st->level_count[idx.index[i]] = sum;
+    }
 }
 // hull record initial values: min-key, max-key, zero-sign lb, zero-sign ub
 __global__ void k_init_hull(unsigned long long* p, unsigned long long n_records, unsigned long long stride) {
@@ -286,6 +317,14 @@ struct DevList {
         dev::BoxList v;
         v.lb = lb; v.ub = ub; v.depth = depth; v.origin = origin; v.leaf = leaf;
         v.stride = cap; v.cap = cap; v.count = counter;
+        v.seg_cap = cap; v.segs = 1;
+        return v;
+    }
+    // The list in segments, with the segments' counters from `counters` on.
+    dev::BoxList segmented(unsigned long long* counters) const {
+        dev::BoxList v = view(counters);
+        v.seg_cap = cap / dev::kSegs;
+        v.segs = dev::kSegs;
         return v;
     }
 };
@@ -334,6 +373,8 @@ struct sqd_core {
     std::size_t state_bytes = 0;
     unsigned long long* d_hull = nullptr;
     unsigned clean = 0;               // jobs (from 0) whose hull records and count slots are known reset
+    sqd::SegCounters segs{nullptr, 0};   // (job) counters of the segmented level lists (none: dense lists)
+    sqd::SegIndex seg_index{};           // their (mode, level)s
     unsigned char* d_has = nullptr;
     sqd::DevList stack, lvl[2], fin, spl, crit, scratch;
     std::uint64_t device_bytes = 0;  // device memory allocated by sqd_core_create
@@ -457,13 +498,23 @@ void set_count(sqd_core* c, unsigned long long* p, unsigned long long v) {
 void reset_state(sqd_core* c) {
     launch(c, KIND_SET_COUNT, "k_state_reset", [&] {
         hipLaunchKernelGGL(k_state_reset, dim3(1, c->ny), dim3(256), 0, c->stream, reinterpret_cast<unsigned long long*>(c->d_state),
-                           static_cast<unsigned long long>(c->state_bytes / sizeof(unsigned long long)), c->job_stride);
+                           static_cast<unsigned long long>(c->state_bytes / sizeof(unsigned long long)), c->segs, c->job_stride);
+        return hipGetLastError();
+    });
+}
+// Enqueues the totals of the segmented lists (level_count of the next state copy).
+void enqueue_level_totals(sqd_core* c) {
+    if(c->segs.n_lists == 0) return;
+    launch(c, KIND_SET_COUNT, "k_level_totals", [&] {
+        hipLaunchKernelGGL(k_level_totals, dim3(1, c->ny), dim3(64), 0, c->stream, c->d_state, c->segs, c->seg_index,
+                           c->job_stride);
         return hipGetLastError();
     });
 }
 // Enqueues the fold of the count slots into the counters and the copy of the
 // device state (of every job of the launches' rows) to its pinned host copy.
 void enqueue_state_copy(sqd_core* c) {
+    if(c->profiling) enqueue_level_totals(c);
     launch(c, KIND_SET_COUNT, "k_fold_counts", [&] {
         const unsigned blocks = static_cast<unsigned>((c->n_slots + kFoldThreads - 1) / kFoldThreads);
         hipLaunchKernelGGL(k_fold_counts, dim3(blocks, c->ny), dim3(kFoldThreads), 0, c->stream, c->d_state, c->d_slots, c->n_slots,
@@ -573,6 +624,15 @@ dev::LevelArgs level_args(sqd_core* c, const dev::BoxList& in, const unsigned lo
     return a;
 }
 
+// Level buffer `which` as the output list of (mode, level): in segments where the
+// core has counters for it, else dense.
+dev::BoxList level_list(sqd_core* c, int which, int mode, int level) {
+    for(unsigned i = 0; i < c->segs.n_lists; ++i)
+        if(c->seg_index.index[i] == mode * 16 + level)
+            return c->lvl[which].segmented(c->segs.p + static_cast<std::size_t>(i) * dev::kSegs * dev::kSegStride);
+    return c->lvl[which].view(&c->d_state->level_count[mode * 16 + level]);
+}
+
 // Static level L of `mode` over the inputs [*base, *base + *count) of `in`
 // (base may be null: 0), at most `max_items` of them, writing `out`.  Its
 // undecided-list counter undec_count[mode * 16 + L] must be zero on entry.
@@ -595,8 +655,8 @@ void run_static_level(sqd_core* c, int mode, int L, const dev::BoxList& in, cons
 // Static levels over the inputs [*base, *base + *count) of `in` (base may be
 // null: 0), at most `max_items` of them.  NONFINAL joins the leaves into d_hull;
 // FINAL appends critical leaves to `crit_out`.  Level L writes lvl[L % 2] with
-// the counter level_count[mode * 16 + L], which must be zero on entry.  With
-// `levels` >= 0 only the first `levels` levels run.
+// the counter level_count[mode * 16 + L], which must be zero on entry (with its
+// segments' counters).  With `levels` >= 0 only the first `levels` levels run.
 void run_static(sqd_core* c, int mode, const dev::BoxList& in, const unsigned long long* base,
                 const unsigned long long* count, unsigned long long max_items, const dev::BoxList& crit_out,
                 int levels = -1) {
@@ -608,7 +668,7 @@ void run_static(sqd_core* c, int mode, const dev::BoxList& in, const unsigned lo
     unsigned long long items = max_items;
     for(int L = 0; L < upto; ++L) {
         const bool last = (L == S - 1);
-        dev::BoxList out = last ? crit_out : c->lvl[L % 2].view(&c->d_state->level_count[mode * 16 + L]);
+        dev::BoxList out = last ? crit_out : level_list(c, L % 2, mode, L);
         run_static_level(c, mode, L, prev, prev_base, prev_count, items, out);
         const unsigned long long children = items * c->st_subs[static_cast<std::size_t>(L)];
         prev = out;
@@ -628,7 +688,7 @@ void run_dynamic(sqd_core* c, int mode, const dev::BoxList& in, const unsigned l
     unsigned long long items = max_items;
     for(int J = 0; J < D; ++J) {
         const bool last = (J == D - 1);
-        dev::BoxList o = last ? out : c->lvl[J % 2].view(&c->d_state->level_count[mode * 16 + J]);
+        dev::BoxList o = last ? out : level_list(c, J % 2, mode, J);
         o.origin = nullptr;
         o.leaf = nullptr;
         dev::BoxList src = prev;
@@ -693,7 +753,7 @@ void begin_call(sqd_core* c) {
 void end_call(sqd_core* c) { c->clean = c->ny; }
 void levels_reset(sqd_core* c) {
     launch(c, KIND_SET_COUNT, "k_levels_reset", [&] {
-        hipLaunchKernelGGL(k_levels_reset, dim3(1), dim3(64), 0, c->stream, c->d_state);
+        hipLaunchKernelGGL(k_levels_reset, dim3(1), dim3(64), 0, c->stream, c->d_state, c->segs);
         return hipGetLastError();
     });
 }
@@ -740,7 +800,7 @@ void enqueue_initial_queue(sqd_core* c, bool only_flagged = false) {
         hipLaunchKernelGGL(k_proof_start, dim3(1, c->ny), dim3(64), 0, c->stream,
                            reinterpret_cast<unsigned long long*>(c->d_state), words, c->d_box_init, c->N, c->scratch.lb,
                            c->scratch.ub, c->scratch.depth, c->scratch.cap, count_word,
-                           only_flagged ? c->d_range + 2 : nullptr, c->job_stride);
+                           only_flagged ? c->d_range + 2 : nullptr, c->segs, c->job_stride);
         return hipGetLastError();
     });
     run_dynamic(c, dev::INIT, c->scratch.view(), c->scratch.count, 1, c->stack.view());
@@ -804,7 +864,7 @@ void enqueue_round(sqd_core* c) {
     DeviceState* st = c->d_state;
     launch(c, KIND_SET_COUNT, "k_round_begin", [&] {
         hipLaunchKernelGGL(k_round_begin, dim3(1, c->ny), dim3(64), 0, c->stream, st, c->k_max, c->stack.cap,
-                           c->split_fanout, c->job_stride);
+                           c->split_fanout, c->segs, c->job_stride);
         return hipGetLastError();
     });
     const unsigned long long K = c->k_max;   // bound on the round's size
@@ -843,6 +903,8 @@ dev::BoxList list_from(const dev::BoxList& l, unsigned long long off, unsigned l
     if(l.origin) v.origin = l.origin + off;
     if(l.leaf) v.leaf = l.leaf + off;
     v.cap = l.cap > off ? l.cap - off : 0;
+    v.seg_cap = v.cap;
+    v.segs = 1;
     v.count = count;
     return v;
 }
@@ -868,14 +930,20 @@ void drain_criticals(sqd_core* c, unsigned long long k, unsigned long long n_fin
         const int S = c->ks->NSTAT;
         const unsigned long long cap = c->crit.cap;
         dev::BoxList src = c->fin.view();
-        unsigned long long n_in = std::min<unsigned long long>(n_fin, c->fin.cap);
+        // the inputs of the last pass: ranges (first entry, entries) of `src`
+        std::vector<std::pair<unsigned long long, unsigned long long>> ranges{{0ull, std::min<unsigned long long>(n_fin, c->fin.cap)}};
         if(S >= 2) {
             levels_reset(c);
-            run_static(c, dev::FINAL, c->fin.view(), nullptr, c->fin.count, n_in, c->crit.view(), S - 1);
-            n_in = read_state(c).level_count[dev::FINAL * 16 + S - 2];
-            src = c->lvl[(S - 2) % 2].view();
+            run_static(c, dev::FINAL, c->fin.view(), nullptr, c->fin.count, ranges[0].second, c->crit.view(), S - 1);
+            src = level_list(c, (S - 2) % 2, dev::FINAL, S - 2);
+            std::vector<unsigned long long> n(static_cast<std::size_t>(src.segs - 1) * dev::kSegStride + 1);
+            hip_check(hipMemcpyAsync(n.data(), src.count, n.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost,
+                                     c->stream), "copy segment counters");
+            read_state(c);
+            ranges.clear();
+            for(unsigned g = 0; g < src.segs; ++g)
+                ranges.push_back({g * src.seg_cap, std::min(n[static_cast<std::size_t>(g) * dev::kSegStride], src.seg_cap)});
         }
-        n_in = std::min(n_in, src.cap);
         // a part's children must fit the critical list and, on a prefiltered or
         // grouped last level, the undecided list; without static levels a part
         // is at most a round's final list
@@ -883,11 +951,12 @@ void drain_criticals(sqd_core* c, unsigned long long k, unsigned long long n_fin
         const unsigned long long room = c->undec_cap ? std::min(cap, c->undec_cap) : cap;
         unsigned long long per = std::max<unsigned long long>(1, room / subs);
         if(S == 0) per = std::min(per, c->k_max);
-        for(unsigned long long off = 0; off < n_in; off += per) {
-            const unsigned long long m = std::min(per, n_in - off);
+        for(const auto& range : ranges)
+        for(unsigned long long off = 0; off < range.second; off += per) {
+            const unsigned long long m = std::min(per, range.second - off);
             set_count(c, &st->part_n, m);
             set_count(c, c->crit.count, 0);
-            const dev::BoxList part = list_from(src, off, &st->part_n);
+            const dev::BoxList part = list_from(src, range.first + off, &st->part_n);
             if(S == 0) {
                 launch(c, KIND_FINAL_NOSTATIC, "final", [&] {
                     return c->ks->final_nostatic(part, c->crit.view(), c->d_discard,
@@ -1034,7 +1103,7 @@ void configure_core(sqd_core* c, int device, const sqd_program* program, const s
 
     // level buffers hold the survivors of one level; size K for the worst case
     const unsigned long long per_entry = 16ull * static_cast<unsigned long long>(c->N) + 12ull;
-    const unsigned long long lvl_cap = std::max<unsigned long long>(1024, s.level_bytes / per_entry);
+    unsigned long long lvl_cap = std::max<unsigned long long>(1024, s.level_bytes / per_entry);
     unsigned long long worst_static = 1, worst_split = 1;
     for(std::size_t L = 0; L + 1 < c->st_subs.size(); ++L) worst_static = std::max<unsigned long long>(worst_static, product(c->st_subs, L + 1));
     for(std::size_t J = 0; J + 1 < c->dyn_subs.size(); ++J) worst_split = std::max<unsigned long long>(worst_split, product(c->dyn_subs, J + 1));
@@ -1042,8 +1111,33 @@ void configure_core(sqd_core* c, int device, const sqd_program* program, const s
     if(worst_init > lvl_cap) throw Failure(SQD_ERR_CAPACITY, "initial queue levels do not fit the level buffers");
     c->split_fanout = product(c->dyn_subs, c->dyn_subs.size());
     unsigned long long kmax = s.dequeue_buffer_size ? s.dequeue_buffer_size : 8192;
-    kmax = std::min(kmax, lvl_cap / worst_static);
-    kmax = std::min(kmax, lvl_cap / worst_split);
+    // Level lists in segments (dev::BoxList): a segment receives at most its
+    // share of a level's children and two waves more, so the lists keep that
+    // much room; buffers too small for it hold dense lists.  The counters come
+    // out of the level buffers' bytes.
+    unsigned n_lists = 0;
+    for(int mode : {dev::NONFINAL, dev::FINAL})
+        for(std::size_t L = 0; L + 1 < c->st_subs.size() && n_lists < sizeof(SegIndex); ++L)
+            c->seg_index.index[n_lists++] = static_cast<unsigned char>(mode * 16 + static_cast<int>(L));
+    for(int mode : {dev::SPLIT, dev::INIT})
+        for(std::size_t J = 0; J + 1 < c->dyn_subs.size() && n_lists < sizeof(SegIndex); ++J)
+            c->seg_index.index[n_lists++] = static_cast<unsigned char>(mode * 16 + static_cast<int>(J));
+    const unsigned long long counter_words = static_cast<unsigned long long>(n_lists) * dev::kSegs * dev::kSegStride;
+    // (a group-tested level that is not the last spreads its survivors by the
+    // place of their parents, which evens out only within each input segment)
+    const unsigned before_last = used >> 1;
+    const unsigned long long slack = 64ull * dev::kSegs * ((s.group_levels & before_last) ? dev::kSegs + 2 : 2);
+    const unsigned long long counter_entries = (counter_words * sizeof(unsigned long long) + 512 + per_entry - 1) / per_entry;
+    unsigned long long room = lvl_cap;   // entries the rounds may fill
+    if(n_lists > 0 && lvl_cap < (1ull << 32) && lvl_cap > counter_entries + slack &&
+       (lvl_cap - counter_entries - slack) / std::max(worst_static, worst_split) >= 1 &&
+       lvl_cap - counter_entries - slack >= worst_init) {
+        c->segs.n_lists = n_lists;
+        lvl_cap -= counter_entries;
+        room = lvl_cap - slack;
+    }
+    kmax = std::min(kmax, room / worst_static);
+    kmax = std::min(kmax, room / worst_split);
     // the FP32 prefilter and the binary64 group test list the children they
     // leave undecided (8 bytes each, level_bytes of them), up to all children
     // of the level, so a round is bounded by the largest such level's children
@@ -1071,6 +1165,7 @@ void configure_core(sqd_core* c, int device, const sqd_program* program, const s
     const unsigned long long stack_cap = std::max<unsigned long long>(s.frontier_capacity, prog.initial_queue_size + 1);
     c->stack.lay(lay, c->N, stack_cap, true, false);
     for(auto& l : c->lvl) l.lay(lay, c->N, lvl_cap, true, true);
+    if(c->segs.n_lists) lay.take(c->segs.p, static_cast<std::size_t>(counter_words));
     c->fin.lay(lay, c->N, kmax, true, false);
     c->spl.lay(lay, c->N, kmax, true, false);
     c->crit.lay(lay, c->N, s.critical_capacity, false, false);
@@ -1091,7 +1186,7 @@ void configure_core(sqd_core* c, int device, const sqd_program* program, const s
     c->job_stride = lay.stride();
     // the sizing rules the level kernels rely on (they also clamp their input
     // counts to the list capacities)
-    if(kmax > c->fin.cap || kmax > c->spl.cap || kmax * worst_static > lvl_cap || kmax * worst_split > lvl_cap ||
+    if(kmax > c->fin.cap || kmax > c->spl.cap || kmax * worst_static > room || kmax * worst_split > room ||
        (c->undec_cap && kmax * worst_undec > c->undec_cap))
         throw Failure(SQD_ERR_INTERNAL, "core sizing rule violated");
 }
