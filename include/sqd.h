@@ -370,7 +370,9 @@ typedef struct sqd_job_result {
     double run_seconds;           /* start to completion */
     double latency_seconds;       /* submission to completion */
     int32_t status;               /* SQD_OK or the job's error */
-    uint32_t joined_running;      /* 1: the job joined a batch that was already running */
+    uint32_t joined_running;      /* 1: the job joined a batch that was already running (a batch
+                                     stays open for 20 ms after its last job while nothing else
+                                     is queued) */
     uint64_t frontier_peak;       /* most cuboids its frontier held after a round */
 } sqd_job_result;
 void sqd_service_options_default(sqd_service_options* options);

@@ -53,6 +53,12 @@ constexpr int static_level_waves() {
     return SQD_LEVEL_WAVES_PER_EU > 0 ? SQD_LEVEL_WAVES_PER_EU : (P::level_waves(L) > 0 ? P::level_waves(L) : 1);
 }
 
+// The kernel with the group test holds both the test and the per-child decision;
+// left to the compiler More2's takes 262 VGPRs and one wave per SIMD.  3 waves:
+// More2's level 733 -> 481 us, the others within 2%; 4 waves spill (More1 42 ->
+// 174 ms).
+constexpr int kGroupWaves = 3;
+
 enum Mode : int { NONFINAL = 0, FINAL = 1, SPLIT = 2, INIT = 3 };
 // Hoisted-term struct of a program without static levels.
 struct NoHoist {};
@@ -279,25 +285,6 @@ __device__ __forceinline__ bool propagate(Num (&lb)[P::N], Num (&ub)[P::N], int 
     return false;
 }
 
-// The inline first step of propagate<P, true> alone: the initial bounds of a
-// change to `arg`, applied in queue order until the first one that changes the
-// box.  -1: a bound emptied the box (propagate returns true); 0: none changed it
-// and the propagation is over with this box (as in propagate); 1: one changed
-// it, and only propagate itself, from the start, gives the propagated box.
-template<class P, class Num>
-__device__ __forceinline__ int propagate_initial(Num (&lb)[P::N], Num (&ub)[P::N], int arg, const Num* C) {
-    constexpr int NB = P::NB;
-    if(NB == 0) return 0;
-    int m = 0;
-    P::deps(arg * 3 + 2, [&](int) { ++m; });
-    if(m >= NB) return 0;   // a full queue reads as empty: nothing is applied
-    int r_first = 0;
-    P::deps(arg * 3 + 2, [&](int k) {
-        if(r_first == 0) r_first = P::apply(k, lb, ub, C);
-    });
-    return r_first < 0 ? -1 : (r_first > 0 ? 1 : 0);
-}
-
 // ---------------------------------------------------------------- wave helpers
 __device__ __forceinline__ unsigned long long wave_append(bool flag, unsigned long long* counter) {
     const unsigned long long mask = __ballot(flag);
@@ -389,6 +376,7 @@ template<bool SEG>
 struct Inputs {
     bool dense;
     unsigned before;                    // segmented lists hold less than 2^32 entries
+    const unsigned* table;              // the sums in LDS
     unsigned long long base, n, seg_cap;
     // The list entry of input `item`, for items that do not decrease over the
     // lanes; called by every lane of the wave (`valid` marks those that need it).
@@ -411,6 +399,16 @@ struct Inputs {
         }
         return at;
     }
+    // The same for items in any order.
+    __device__ __forceinline__ unsigned long long entry_any(unsigned long long item64) const {
+        if(!SEG || dense) return base + item64;
+        const unsigned item = static_cast<unsigned>(item64);
+        unsigned g = 0;
+#pragma unroll
+        for(unsigned step = kSegs / 2; step > 0; step >>= 1)
+            if(table[g + step] <= item) g += step;
+        return g * seg_cap + (item - table[g]);
+    }
 };
 // v plus the value SHIFT lanes below (0 past the row's first lane) in rows of 16 lanes.
 template<int SHIFT> __device__ __forceinline__ unsigned row_add(unsigned v) {
@@ -424,6 +422,7 @@ __device__ __forceinline__ Inputs<SEG> level_inputs(const LevelArgs& a) {
     in.base = a.in_base ? *a.in_base : 0ull;
     in.dense = true;
     in.before = 0;
+    in.table = nullptr;
     if constexpr(SEG) {
         static_assert(kSegs == 16, "the scan covers one row of 16 lanes");
         in.dense = a.in.segs <= 1;
@@ -439,6 +438,7 @@ __device__ __forceinline__ Inputs<SEG> level_inputs(const LevelArgs& a) {
                 s_before[threadIdx.x] = threadIdx.x < kSegs ? sum - v : __builtin_amdgcn_readlane(sum, kSegs - 1);
             }
             __syncthreads();
+            in.table = s_before;
             in.before = s_before[__lane_id()];
             in.n = __builtin_amdgcn_readlane(in.before, kSegs);
             return in;
@@ -458,6 +458,21 @@ __device__ __forceinline__ unsigned long long list_append(const BoxList& l, bool
     const unsigned s = !SEG || l.segs <= 1 ? 0u : seg % kSegs;
     const unsigned long long pos = wave_append(flag, l.count + static_cast<unsigned long long>(s) * kSegStride);
     return pos < l.seg_cap ? s * l.seg_cap + pos : ~0ull;
+}
+
+// The same with a segment per lane.
+template<bool SEG>
+__device__ __forceinline__ unsigned long long list_append_mixed(const BoxList& l, bool flag, unsigned seg) {
+    if(!SEG || l.segs <= 1) return list_append<SEG>(l, flag, 0u);
+    unsigned long long pos = ~0ull;
+    for(unsigned long long m = __ballot(flag); m;) {
+        const unsigned s = __shfl(seg % kSegs, __ffsll(static_cast<long long>(m)) - 1);
+        const bool now = flag && seg % kSegs == s;
+        const unsigned long long at = list_append<SEG>(l, now, s);
+        if(now) pos = at;
+        m &= ~__ballot(now);
+    }
+    return pos;
 }
 
 template<class P>
@@ -561,6 +576,25 @@ __device__ __forceinline__ int group_size(const LevelArgs& args, unsigned long l
     return 1;
 }
 
+// Children per group of k_static_grouped's first test (a power of two dividing
+// SUBS): as args.children_per_lane asks, else up to 32.  Proof times at 8 / 16 /
+// 32: One 87 / 84 / 86 us, Two 160 / 135 / 127 us, Three 202 / 192 / 186 us, More1
+// 49 / 49 / 50 ms; 64 was slower for One.  A launch whose children fit one trip
+// of its lanes decides them at once: a test would come before the same decision.
+constexpr int kMaxGroup = 64;
+template<int SUBS, int CPL>
+__device__ __forceinline__ int plain_group_size(const LevelArgs& args, unsigned long long n_items, unsigned long long stride) {
+    if(n_items * static_cast<unsigned long long>(SUBS) <= stride) return 1;
+    int c = CPL;
+    const int want = args.children_per_lane > 0 ? args.children_per_lane : 32;
+    while(c > want) c >>= 1;
+    return c;
+}
+// Neighbouring groups that a trip of k_static_grouped takes together.  Fewer
+// spread the work more evenly (More1's level at 16 / 8 / 4 / 1: 52 / 46 / 42 / 37
+// ms), more load whole lines (Four's 205 / 208 / 215 / 329 us).
+constexpr unsigned kRun = 4;
+
 // Child w of a static level, counted over the entries of its input list: the
 // parent box at entry w / SUBS with the level's variable replaced by subrange
 // w % SUBS of the splitter (splitter.hpp:44-59), its dynamic cuboid (origin) and
@@ -587,8 +621,8 @@ __device__ __forceinline__ void static_child(const LevelArgs& args, const Inputs
 // non-final level), record a critical (last final level) or append the survivor
 // to the next level's list.  Called by every lane of the wave (the hull join and
 // the append are wave-wide); `valid` marks the lanes that hold a child, `seg` is
-// the output segment of the wave's survivors.
-template<class P, int MODE, int L>
+// the output segment of the wave's survivors (MIXED: of the lane's).
+template<class P, int MODE, int L, bool MIXED = false>
 __device__ __forceinline__ void static_decide(const LevelArgs& args, const Inputs<(L > 0)>& in, bool valid,
                                               unsigned long long w, unsigned seg, const double* s_c, PropScratch<P>& s_prop,
                                               unsigned long long& c_leaf, unsigned long long& c_crit) {
@@ -614,7 +648,7 @@ __device__ __forceinline__ void static_decide(const LevelArgs& args, const Input
     }
     if(LAST && MODE == NONFINAL) hull_join<N>(args.hull, join, origin, leaf, lb, ub);
     if(!LAST || MODE == FINAL) {
-        const unsigned long long pos = list_append<!LAST>(args.out, survive, seg);
+        const unsigned long long pos = MIXED ? list_append_mixed<!LAST>(args.out, survive, seg) : list_append<!LAST>(args.out, survive, seg);
         if(survive) {
             if(pos != ~0ull) {
                 store_box<P>(args.out, pos, lb, ub);
@@ -627,104 +661,15 @@ __device__ __forceinline__ void static_decide(const LevelArgs& args, const Input
             }
         }
     }
-}
-
-// The binary64 decision of child i of the parent (plb, pub), whose terms free
-// of the level's variable were hoisted into h (in LDS): as static_decide, but
-// the rows are checked with the hoisted terms when propagation left every other
-// variable bit for bit as in the parent (the child's box is then, in every
-// variable those terms read, the box h was computed for), and in full otherwise.
-// DEFER: the child is decided here only when the level's initial bounds leave
-// the box unchanged (then the hoisted terms apply) or empty it; otherwise
-// `defer` is set and nothing is counted or written for it: the caller decides
-// it later with static_decide, together with other such children.
-// Called by every lane of the wave.
-template<class P, int MODE, int L, bool DEFER>
-__device__ __forceinline__ void static_decide_hoisted(const LevelArgs& args, bool valid, const double (&plb)[P::N],
-                                                      const double (&pub)[P::N], double pl, double pu, double wd, int i,
-                                                      unsigned origin, unsigned leaf,
-                                                      const typename P::template Hoist<L, double>& h,
-                                                      unsigned seg, const double* s_c, PropScratch<P>& s_prop,
-                                                      unsigned long long& c_leaf, unsigned long long& c_crit,
-                                                      bool& defer) {
-    constexpr int N = P::N;
-    constexpr int ARG = P::st_arg(L);
-    constexpr int SUBS = P::st_subs(L);
-    constexpr bool LAST = (L == P::NSTAT - 1);
-    bool survive = false, join = false;
-    double lb[N], ub[N];
-#pragma unroll
-    for(int a = 0; a < N; ++a) { lb[a] = plb[a]; ub[a] = pub[a]; }
-    defer = false;
-    if(valid) {
-        lb[ARG] = split_point(pl, pu, wd, i, SUBS);
-        ub[ARG] = split_point(pl, pu, wd, i + 1, SUBS);
-        bool pruned;
-        if constexpr(DEFER) {
-            const int r = propagate_initial<P>(lb, ub, ARG, s_c);
-            pruned = r < 0;
-            defer = r > 0;
-        } else {
-            pruned = propagate<P, P::prop_fast(L)>(lb, ub, ARG, N, 4u, s_c, s_prop);
-        }
-        if(defer) {
-        } else if(pruned) {
-            ++c_leaf;
-        } else {
-            // with DEFER the box is the parent's apart from the level's variable
-            bool same = true;
-#pragma unroll
-            for(int a = 0; a < N; ++a)
-                if(!DEFER && a != ARG) same = same && bits(lb[a]) == bits(plb[a]) && bits(ub[a]) == bits(pub[a]);
-            const bool violated = same ? P::template rows_violated_hoisted<L>(lb, ub, s_c, h)
-                                       : P::template rows_violated<L>(lb, ub, s_c);
-            if(violated) {
-                ++c_leaf;
-            } else if(LAST) {
-                ++c_leaf;
-                if(MODE == FINAL) { ++c_crit; survive = true; }
-                else join = true;
-            } else {
-                survive = true;
-            }
-        }
-    }
-    if(LAST && MODE == NONFINAL) hull_join<N>(args.hull, join, origin, leaf, lb, ub);
-    if(!LAST || MODE == FINAL) {
-        const unsigned long long pos = list_append<!LAST>(args.out, survive, seg);
-        if(survive) {
-            if(pos != ~0ull) {
-                store_box<P>(args.out, pos, lb, ub);
-                if(args.out.origin) { args.out.origin[pos] = origin; args.out.leaf[pos] = leaf; }
-            } else if(!LAST) {
-                // a level list is sized so that this cannot happen; the critical
-                // list's count keeps going past its capacity, which the host
-                // compares with it (and then repeats the final pass in parts)
-                atomicAdd(&args.counters->overflow, 1ull);
-            }
-        }
-    }
-}
-
-// Whether the binary64 static level L hoists its split-free terms per wave:
-// when a wave can take all children of a parent in several trips of 64, the
-// level has such terms, and it is not the first static level (whose parents,
-// the round's dynamic cuboids, are usually too few to give every wave one).
-template<class P, int L>
-constexpr bool wave_hoisting() {
-    return L >= 1 && P::st_subs(L) % 64 == 0 && P::st_subs(L) >= 128 &&
-           sizeof(typename P::template Hoist<L, double>) > 1;
 }
 
 // Level L of the static grid (modes NONFINAL and FINAL).
 //
-// F32 = false: every child w of the level's parents is decided in binary64.
-// Where wave_hoisting<P, L>() holds, each wave takes whole parents: it computes
-// the parent's split-free terms once into its LDS slot, then decides the
-// SUBS children in trips of 64 (static_decide_hoisted).
+// F32 = false: every child w of the level's parents is decided in binary64 (the
+// levels before the last, whose children mostly survive, so that a group test
+// would be one evaluation more).
 // F32 = true: the children listed in args.undec (by k_static_prefilter, those
-// binary32 left undecided; by k_static_group64, those of the groups that passed
-// the group test) are decided in binary64, exactly as above.
+// binary32 left undecided) are decided in binary64, exactly as above.
 template<class P, int MODE, int L, bool F32>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(static_level_waves<P, L>())))
 void k_static_level(LevelArgs job0) {
@@ -739,12 +684,9 @@ void k_static_level(LevelArgs job0) {
     const unsigned long long total =
         F32 ? (listed < args.undec_cap ? listed : args.undec_cap) : n_items * static_cast<unsigned long long>(SUBS);
     const unsigned long long first = static_cast<unsigned long long>(blockIdx.x) * blockDim.x + threadIdx.x;
-    // a block without inputs leaves at once (block-uniform: no barrier is skipped
-    // by part of a block, and it has no counts to add); the hoisting path hands
-    // out whole parents per wave
-    if(!F32 && wave_hoisting<P, L>() ? static_cast<unsigned long long>(blockIdx.x) * (blockDim.x / 64) >= n_items
-                                     : static_cast<unsigned long long>(blockIdx.x) * blockDim.x >= total)
-        return;
+    // a block without children leaves at once (block-uniform: no barrier is skipped
+    // by part of a block, and it has no counts to add)
+    if(static_cast<unsigned long long>(blockIdx.x) * blockDim.x >= total) return;
     // the generated code takes the constants as literals (P::kc) and does not
     // read the array pointer its functions take
     const double* const s_c = nullptr;
@@ -754,101 +696,21 @@ void k_static_level(LevelArgs job0) {
     unsigned long long c_cub = 0, c_leaf = 0, c_crit = 0;
     // every lane of a wave runs the same number of loop trips, so the wave-wide
     // ballots always see all lanes of the wave
-    if constexpr(!F32 && wave_hoisting<P, L>()) {
-        constexpr int N = P::N;
-        constexpr int ARG = P::st_arg(L);
-        using H = typename P::template Hoist<L, double>;
-        __shared__ H s_h[kBlock / 64];
-        // the wave's loop state is the same on all its lanes: in scalar
-        // registers it leaves the vector registers to the deferred children's
-        // full decision, which spills otherwise
-        const unsigned wib = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);   // wave in block
-        H& h = s_h[wib];
-        // Children whose initial bounds change another variable (a few percent;
-        // they need the full propagation and the full rows) are listed per wave
-        // and decided 64 at a time, so that a wave does not run that path for
-        // one or two of its lanes.  The list holds fewer than 64 children
-        // between parents, so 64 + SUBS entries suffice.
-        constexpr bool DEFER = P::prop_fast(L) && L == P::NSTAT - 1;
-        __shared__ unsigned long long s_def[kBlock / 64][DEFER ? 64 + SUBS : 1];
-        unsigned long long* const dq = s_def[wib];
-        unsigned dcount = 0;   // wave-uniform
-        const int lane = static_cast<int>(__lane_id());
-        const unsigned long long below = (1ull << lane) - 1ull;
-        const unsigned long long waves = static_cast<unsigned long long>(gridDim.x) * (blockDim.x / 64);
-        const unsigned long long wave = static_cast<unsigned long long>(blockIdx.x) * (blockDim.x / 64) + wib;
-        const unsigned long long items = wave_uniform(n_items);
-        const unsigned long long wtrips = (items + waves - 1) / waves;   // the same for every wave
-        for(unsigned long long trip = 0; trip < wtrips; ++trip) {
-            const unsigned long long item = wave + trip * waves;
-            const bool valid = item < items;                              // wave-uniform
-            const unsigned long long src = wave_uniform(in.entry(item, valid));
-            double plb[N], pub[N];
-            double pl = 0, pu = 0, wd = 0;
-            unsigned p_origin = 0, p_leaf = 0;
-#pragma unroll
-            for(int a = 0; a < N; ++a) { plb[a] = 0.0; pub[a] = 0.0; }
-            if(valid) {
-                load_box<P>(args.in, src, plb, pub);
-                if(args.in.origin) { p_origin = args.in.origin[src]; p_leaf = args.in.leaf[src]; }
-                else { p_origin = static_cast<unsigned>(item); p_leaf = 0; }
-                pl = plb[ARG];
-                pu = pub[ARG];
-                wd = split_width(pl, pu, SUBS);
-                H hv;
-                P::template hoist<L>(plb, pub, s_c, hv);
-                if(lane == 0) { h = hv; c_cub += SUBS; }
-            }
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-#pragma unroll 1
-            for(int k = 0; k < SUBS / 64; ++k) {
-                const int i = lane + 64 * k;
-                bool defer;
-                static_decide_hoisted<P, MODE, L, DEFER>(args, valid, plb, pub, pl, pu, wd, i, p_origin,
-                                                         p_leaf * SUBS + static_cast<unsigned>(i), h,
-                                                         static_cast<unsigned>(item) * (SUBS / 64) + k, s_c, s_prop,
-                                                         c_leaf, c_crit, defer);
-                if constexpr(DEFER) {
-                    const unsigned long long m = __ballot(defer);
-                    if(defer) dq[dcount + __popcll(m & below)] = src * SUBS + static_cast<unsigned>(i);
-                    dcount += static_cast<unsigned>(__popcll(m));
-                }
-            }
-            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            if constexpr(DEFER) {
-                // full trips of 64 while the list holds them; after the last
-                // parent, the rest
-                const bool last = trip + 1 == wtrips;
-                while(dcount >= 64 || (last && dcount > 0)) {
-                    const unsigned take = dcount >= 64 ? 64u : dcount;
-                    dcount -= take;
-                    const bool v = static_cast<unsigned>(lane) < take;
-                    const unsigned long long w = v ? dq[dcount + lane] : 0ull;
-                    static_decide<P, MODE, L>(args, in, v, w, 0u, s_c, s_prop, c_leaf, c_crit);
-                }
-                __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-            }
+    const unsigned long long trips = (total + stride - 1) / stride;
+    for(unsigned long long trip = 0; trip < trips; ++trip) {
+        const unsigned long long t = first + trip * stride;
+        const bool valid = t < total;
+        unsigned long long w = 0;
+        if(F32) {
+            if(valid) w = args.undec[t];
+        } else {
+            w = in.entry(t / SUBS, valid) * SUBS + t % SUBS;
+            if(valid && t % SUBS == 0) c_cub += SUBS;
         }
-    } else {
-        const unsigned long long trips = (total + stride - 1) / stride;
-        for(unsigned long long trip = 0; trip < trips; ++trip) {
-            const unsigned long long t = first + trip * stride;
-            const bool valid = t < total;
-            unsigned long long w = 0;
-            if(F32) {
-                if(valid) w = args.undec[t];
-            } else {
-                w = in.entry(t / SUBS, valid) * SUBS + t % SUBS;
-                if(valid && t % SUBS == 0) c_cub += SUBS;
-            }
-            // successive waves of children append to successive segments, so a
-            // segment receives at most its share of them and one wave more
-            const unsigned seg = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(t / 64));
-            static_decide<P, MODE, L>(args, in, valid, w, seg, s_c, s_prop, c_leaf, c_crit);
-        }
+        // successive waves of children append to successive segments, so a
+        // segment receives at most its share of them and one wave more
+        const unsigned seg = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(t / 64));
+        static_decide<P, MODE, L>(args, in, valid, w, seg, s_c, s_prop, c_leaf, c_crit);
     }
     block_counts_add(args.block_counts, c_cub, c_leaf, MODE == FINAL ? c_crit : 0ull);
 }
@@ -1015,72 +877,137 @@ __global__ __launch_bounds__(kBlock) SQD_LEVEL_ATTR void k_static_prefilter(Leve
     block_counts_add(args.block_counts, c_cub, c_leaf, 0ull, c_dec, c_chk);
 }
 
-// The binary64 group test of static level L (the levels of
-// sqd_settings.group_levels that the FP32 prefilter does not take): each lane
-// checks the rows once, in binary64, on the parent's box with A over a group of
-// cpl consecutive children (the terms free of A hoisted), and appends the
-// children of a group that passes to args.undec; k_static_level<..., true> then
-// decides them one by one exactly as the plain pass does.  The binary64
-// operations are inclusion-isotone where defined (as for the FP32 prefilter's
-// group test) and every child's propagated box lies in the group's box, so a group that fails a row holds only children that the plain
-// pass prunes too (by propagation or by a row): they are counted as its pruned
-// leaves, and survivors, hulls, criticals and counts are exactly the plain
-// pass's.  The test runs in its own kernel so that neither pass carries the
-// other's registers.
+// The binary64 decision of static level L with the group test: what the last
+// static level of a plain proof runs (nearly all of its children fail a row
+// together with their siblings), and the levels of sqd_settings.group_levels.
+//
+// A group is cpl consecutive children of one parent; its box is the parent's with
+// the level's variable over the whole group.  The binary64 operations are
+// inclusion-isotone where defined (as for the FP32 prefilter's group test) and
+// every child's propagated box lies in the group's box, so a group that fails a
+// row holds only children that the per-child decision prunes too (by propagation
+// or by a row): they are counted as its pruned leaves, and survivors, hulls,
+// criticals and counts are exactly those of deciding every child by itself.  The
+// test takes the cheap enclosures of arc cosines, which contain the exact ones.
+//
+// Each wave works on its own: it tests 64 groups at a time, lists the groups left
+// in LDS, tests those again in smaller parts when they are large, and decides the
+// children of what is left 64 at a time (static_decide), so that the long
+// per-child path runs on full waves.  Nothing leaves the kernel but what survives,
+// and a level is one launch.
+//
+// Bound by VALU issue and latency (2 to 3 waves per SIMD).  Against one evaluation
+// per child: One's level 1 (2.8 M children) 75 -> 20 us, Three's (3.3 M) 276 -> 23
+// us, Four's level 2 (33.7 M) 3.43 -> 0.21 ms, More2's (115 M) 14.2 -> 0.48 ms,
+// More1's level 1 (1.01 G over 160 rounds) 258 -> 42 ms.
 template<class P, int MODE, int L>
-__global__ __launch_bounds__(kBlock) SQD_LEVEL_ATTR void k_static_group64(LevelArgs job0) {
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kGroupWaves)))
+void k_static_grouped(LevelArgs job0) {
     const LevelArgs args = job_args(job0);
     constexpr int N = P::N;
     constexpr int ARG = P::st_arg(L);
     constexpr int SUBS = P::st_subs(L);
-    constexpr int CPL = children_per_lane<SUBS>();
+    constexpr int CPL = children_per_lane<SUBS>() < kMaxGroup ? children_per_lane<SUBS>() : kMaxGroup;
     const double* const s_c = nullptr;   // constants are literals in the generated code (P::kc)
-    enter_round_down();
+    __shared__ PropScratch<P> s_prop;
+    // groups left by the first test, in parts (first child), and groups whose
+    // children are to be decided; both hold fewer than 64 children's worth of
+    // groups before a test adds to them
+    __shared__ unsigned long long s_parts[kBlock / 64][64 + 4 * 64], s_left[kBlock / 64][64 + 64];
     const Inputs<(L > 0)> in = level_inputs<(L > 0)>(args);
-    const unsigned long long n_items = in.n;
     const unsigned long long stride = static_cast<unsigned long long>(gridDim.x) * blockDim.x;
-    const int cpl = group_size<SUBS, CPL>(args, n_items, stride);
-    const int step = SUBS / cpl;                                                       // groups per parent
-    const unsigned long long total = n_items * static_cast<unsigned long long>(step);  // groups
-    const unsigned long long first = static_cast<unsigned long long>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if(static_cast<unsigned long long>(blockIdx.x) * blockDim.x >= total) return;   // no groups (block-uniform)
-    const unsigned long long trips = (total + stride - 1) / stride;
-    unsigned long long c_cub = 0, c_leaf = 0;
-    for(unsigned long long trip = 0; trip < trips; ++trip) {
-        const unsigned long long slot = first + trip * stride;
-        const unsigned long long src = in.entry(slot / static_cast<unsigned long long>(step), slot < total);
-        bool keep = false;
-        unsigned long long w0 = 0;
-        if(slot < total) {
-            const int g = static_cast<int>(slot % static_cast<unsigned long long>(step));
-            if(g == 0) c_cub += SUBS;
-            w0 = src * SUBS + static_cast<unsigned long long>(g * cpl);
-            keep = true;
-            if(cpl > 1) {
-                double lb[N], ub[N];
-                load_box<P>(args.in, src, lb, ub);
-                typename P::template Hoist<L, double> h;
-                P::template hoist<L>(lb, ub, s_c, h);
-                const double pl = lb[ARG], pu = ub[ARG];
-                const double wd = split_width(pl, pu, SUBS);
-                lb[ARG] = split_point(pl, pu, wd, g * cpl, SUBS);
-                ub[ARG] = split_point(pl, pu, wd, (g + 1) * cpl, SUBS);
-                if(P::template rows_violated_hoisted<L>(lb, ub, s_c, h)) {
-                    keep = false;
-                    c_leaf += static_cast<unsigned long long>(cpl);
-                }
+    const int cpl = plain_group_size<SUBS, CPL>(args, in.n, stride);
+    const int part = cpl >= 16 ? (cpl > 16 ? cpl / 4 : 8) : cpl;   // size of the groups whose children are decided
+    const unsigned long long total = in.n * static_cast<unsigned long long>(SUBS / cpl);   // groups
+    // A trip takes kRun neighbouring groups at each of 64 / kRun places spread over
+    // the list: neighbours keep many or few of their groups together, and a wave
+    // that got 64 of them could have 30 times the work of another
+    const unsigned long long trips = (total + 63) / 64;
+    if(static_cast<unsigned long long>(blockIdx.x) * (kBlock / 64) >= trips) return;   // no groups (block-uniform)
+    enter_round_down();
+    const unsigned wib = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);   // wave in block
+    unsigned long long* const parts = s_parts[wib];
+    unsigned long long* const left = s_left[wib];
+    const int lane = static_cast<int>(__lane_id());
+    const unsigned long long below = (1ull << lane) - 1ull;
+    const unsigned split = static_cast<unsigned>(cpl / part);    // parts of a group (at most 4)
+    const unsigned per = 64u / static_cast<unsigned>(part);   // listed groups that make 64 children
+    unsigned nq = 0, nl = 0;                                     // wave-uniform list sizes
+    unsigned untested = 0;                                       // trips of groups to leave untested
+    unsigned long long next = static_cast<unsigned long long>(blockIdx.x) * (kBlock / 64) + wib;
+    unsigned long long c_cub = 0, c_leaf = 0, c_crit = 0;
+    for(;;) {
+        const bool more = next < trips;
+        unsigned long long w = 0;   // first child of the lane's group, or the lane's child
+        bool valid, decide;
+        int len = cpl;
+        if(nl >= per || (nl > 0 && !more && nq == 0)) {
+            const unsigned take = nl < per ? nl : per;
+            nl -= take;
+            const unsigned q = static_cast<unsigned>(lane) / static_cast<unsigned>(part);
+            valid = q < take;
+            if(valid) w = left[nl + q] + static_cast<unsigned>(lane) % static_cast<unsigned>(part);
+            decide = true;
+        } else if(nq >= 64 || (nq > 0 && !more)) {
+            const unsigned take = nq < 64u ? nq : 64u;
+            nq -= take;
+            valid = static_cast<unsigned>(lane) < take;
+            if(valid) w = parts[nq + lane];
+            len = part;
+            decide = false;
+        } else if(more) {
+            const unsigned run = static_cast<unsigned>(lane) / kRun;
+            const unsigned long long g = (run * trips + next) * kRun + static_cast<unsigned>(lane) % kRun;
+            valid = g < total;
+            const unsigned step = static_cast<unsigned>(SUBS / cpl);
+            if(valid) {
+                w = in.entry_any(g / step) * SUBS + g % step * static_cast<unsigned>(cpl);
+                c_cub += static_cast<unsigned long long>(cpl);
             }
+            next += stride / 64;
+            decide = cpl == 1;
+        } else {
+            break;
         }
-        const unsigned long long pos = wave_append_n(keep, static_cast<unsigned>(cpl), args.undec_count);
-        if(keep) {
-            if(pos + static_cast<unsigned long long>(cpl) <= args.undec_cap) {
-                for(int k = 0; k < cpl; ++k) args.undec[pos + k] = w0 + static_cast<unsigned long long>(k);
-            } else {
-                atomicAdd(&args.counters->overflow, 1ull);
-            }
+        if(decide) {
+            static_decide<P, MODE, L, true>(args, in, valid, w, static_cast<unsigned>(w / 64), s_c, s_prop, c_leaf, c_crit);
+            continue;
         }
+        bool keep = valid;
+        const bool whole = len != part;
+        if(whole && untested > 0) {
+            --untested;   // straight to the parts
+        } else if(valid) {
+            const int i = static_cast<int>(w % SUBS);
+            double lb[N], ub[N];
+            load_box<P>(args.in, w / SUBS, lb, ub);
+            typename P::template Hoist<L, double> h;
+            P::template hoist<L>(lb, ub, s_c, h);
+            const double pl = lb[ARG], pu = ub[ARG];
+            const double wd = split_width(pl, pu, SUBS);
+            lb[ARG] = split_point(pl, pu, wd, i, SUBS);
+            ub[ARG] = split_point(pl, pu, wd, i + len, SUBS);
+            keep = !P::template rows_violated_hoisted<L>(lb, ub, s_c, h);
+            if(!keep) c_leaf += static_cast<unsigned long long>(len);
+        }
+        const unsigned long long m = __ballot(keep);
+        const unsigned at = static_cast<unsigned>(__popcll(m & below)), n = static_cast<unsigned>(__popcll(m));
+        if(whole) {
+            // a first test that leaves more than three quarters of the groups costs
+            // more than it saves: the next groups go to their parts untested
+            if(untested == 0 && 4u * n > 3u * static_cast<unsigned>(__popcll(__ballot(valid)))) untested = 16;
+            if(keep)
+                for(unsigned k = 0; k < split; ++k) parts[nq + split * at + k] = w + k * static_cast<unsigned>(part);
+            nq += split * n;
+        } else {
+            if(keep) left[nl + at] = w;
+            nl += n;
+        }
+        // the lists are read by other lanes of the wave
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        __builtin_amdgcn_wave_barrier();
     }
-    block_counts_add(args.block_counts, c_cub, c_leaf, 0ull);
+    block_counts_add(args.block_counts, c_cub, c_leaf, MODE == FINAL ? c_crit : 0ull);
 }
 
 // ---------------------------------------------------------------- dynamic levels

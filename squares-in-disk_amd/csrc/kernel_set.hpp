@@ -84,36 +84,34 @@ inline unsigned level_grid(unsigned per_cu, unsigned cus, unsigned jobs, unsigne
     return static_cast<unsigned>(need < 1 ? 1 : (need < most ? need : most));
 }
 
+// One static level in binary64 with the group test.
+template<class P, int MODE, int L>
+hipError_t launch_one_grouped(const dev::LevelArgs& a, unsigned long long max_children, unsigned cus, unsigned grid,
+                              hipStream_t s) {
+    static const unsigned per_cu = blocks_per_cu(dev::k_static_grouped<P, MODE, L>);
+    hipLaunchKernelGGL((dev::k_static_grouped<P, MODE, L>),
+                       dim3(level_grid(per_cu, cus, jobs_of(a), max_children, grid), jobs_of(a)), dim3(dev::kBlock), 0, s, a);
+    return hipGetLastError();
+}
 // One static level: the binary64 kernel over every child, or (F32) the binary32
 // prefilter followed by the binary64 kernel over the children it left undecided.
+// The last level's binary64 kernel is the one with the group test.
 template<class P, int MODE, int L, bool F32>
 hipError_t launch_one_static(const dev::LevelArgs& a, unsigned long long max_children, unsigned cus, unsigned grid,
                              hipStream_t s) {
-    if(F32) {
+    if constexpr(!F32 && L == P::NSTAT - 1) return launch_one_grouped<P, MODE, L>(a, max_children, cus, grid, s);
+    if constexpr(F32) {
         static const unsigned pre_cu = blocks_per_cu(dev::k_static_prefilter<P, MODE, L>);
         hipLaunchKernelGGL((dev::k_static_prefilter<P, MODE, L>), dim3(level_grid(pre_cu, cus, jobs_of(a), max_children, grid), jobs_of(a)),
                            dim3(dev::kBlock), 0, s, a);
         const hipError_t e = hipGetLastError();
         if(e != hipSuccess) return e;
     }
-    static const unsigned per_cu = blocks_per_cu(dev::k_static_level<P, MODE, L, F32>);
-    hipLaunchKernelGGL((dev::k_static_level<P, MODE, L, F32>),
-                       dim3(level_grid(per_cu, cus, jobs_of(a), max_children, grid), jobs_of(a)), dim3(dev::kBlock), 0, s, a);
-    return hipGetLastError();
-}
-// One static level with the binary64 group test: the test, then the binary64
-// kernel over the children of the groups it left.
-template<class P, int MODE, int L>
-hipError_t launch_one_grouped(const dev::LevelArgs& a, unsigned long long max_children, unsigned cus, unsigned grid,
-                              hipStream_t s) {
-    static const unsigned pre_cu = blocks_per_cu(dev::k_static_group64<P, MODE, L>);
-    hipLaunchKernelGGL((dev::k_static_group64<P, MODE, L>),
-                       dim3(level_grid(pre_cu, cus, jobs_of(a), max_children, grid), jobs_of(a)), dim3(dev::kBlock), 0, s, a);
-    const hipError_t e = hipGetLastError();
-    if(e != hipSuccess) return e;
-    static const unsigned per_cu = blocks_per_cu(dev::k_static_level<P, MODE, L, true>);
-    hipLaunchKernelGGL((dev::k_static_level<P, MODE, L, true>),
-                       dim3(level_grid(per_cu, cus, jobs_of(a), max_children, grid), jobs_of(a)), dim3(dev::kBlock), 0, s, a);
+    if constexpr(F32 || L != P::NSTAT - 1) {
+        static const unsigned per_cu = blocks_per_cu(dev::k_static_level<P, MODE, L, F32>);
+        hipLaunchKernelGGL((dev::k_static_level<P, MODE, L, F32>),
+                           dim3(level_grid(per_cu, cus, jobs_of(a), max_children, grid), jobs_of(a)), dim3(dev::kBlock), 0, s, a);
+    }
     return hipGetLastError();
 }
 template<class P, int MODE, int... L>

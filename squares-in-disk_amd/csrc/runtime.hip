@@ -14,6 +14,7 @@
 #include <cstdio>
 #include <cstring>
 #include <functional>
+#include <limits>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -386,6 +387,7 @@ struct sqd_core {
     void* progress_user = nullptr;
     double progress_start = 0, progress_every = 0;
     std::vector<double> head;        // 2N: the frontier's top for progress reports
+    bool groups_valid = true;        // the current call's boxes allow the binary64 group test
     bool fp32 = false;               // some static level runs the FP32-prefiltered kernels
     // sqd_prove as HIP graphs: the initial queue with the first round, and one later round
     hipGraphExec_t g_first = nullptr, g_round = nullptr;
@@ -642,10 +644,16 @@ void run_static_level(sqd_core* c, int mode, int L, const dev::BoxList& in, cons
     if(L == 0) { src.origin = nullptr; src.leaf = nullptr; }  // the input index is the origin
     dev::LevelArgs a = level_args(c, src, base, count, out);
     a.undec_count = &c->d_state->undec_count[mode * 16 + L];
+    // the group test: sized by the settings on the levels that ask for one (here or
+    // in the prefilter), by the kernel on the last level of a plain proof; off
+    // (one child per group) for boxes it is not valid for
+    const bool asked = ((c->settings.fp32_prefilter | c->settings.group_levels) >> L) & 1u;
+    const bool f32 = (c->settings.fp32_prefilter >> L) & 1u;
+    if(!f32 && !c->groups_valid) a.children_per_lane = 1;
+    else if(!asked) a.children_per_lane = 0;
     const unsigned long long children = max_items * c->st_subs[static_cast<std::size_t>(L)];
     launch(c, mode * 16 + L, "static level launch",
            [&] {
-               const bool f32 = (c->settings.fp32_prefilter >> L) & 1u;
                const bool grp = (c->settings.group_levels >> L) & 1u;
                const int m = mode | (f32 ? dev::kModeF32 : grp ? dev::kModeGroup : 0);
                return c->ks->static_level(m, L, a, children, c->cus, c->grid_override, c->stream);
@@ -736,6 +744,7 @@ void download_soa(sqd_core* c, const DevList& l, unsigned long long n, double* l
 // with begin_call and marks the core clean when it completes; after a failed
 // call both are reset in full before the next use.
 void begin_call(sqd_core* c) {
+    c->groups_valid = true;
     // any other computing call ends a continuous batch: its rows' jobs are dropped
     std::fill(c->row_state.begin(), c->row_state.end(), static_cast<unsigned char>(0));
     if(c->clean < c->ny) {
@@ -748,6 +757,22 @@ void begin_call(sqd_core* c) {
         reset_state(c);
     }
     c->clean = 0;   // until the call completes
+}
+// The group test decides like the per-child test where the interval operations
+// are inclusion-isotone: on finite boxes inside the program's compile-time box,
+// whose signs the generated code relies on.  Boxes of a proof always are; for
+// boxes (SoA, stride n) that a caller hands over, this is checked.
+void check_groups_valid(sqd_core* c, const double* lb, const double* ub, std::size_t n) {
+    const auto& prog = c->program->prog;
+    bool ok = true;
+    for(int a = 0; a < c->N; ++a) {
+        const double lo = std::max(prog.box_lb[static_cast<std::size_t>(a)], -std::numeric_limits<double>::max());
+        const double hi = std::min(prog.box_ub[static_cast<std::size_t>(a)], std::numeric_limits<double>::max());
+        const double* l = lb + static_cast<std::size_t>(a) * n;
+        const double* u = ub + static_cast<std::size_t>(a) * n;
+        for(std::size_t i = 0; i < n; ++i) ok = ok & (l[i] >= lo) & (u[i] <= hi) & (l[i] <= u[i]);
+    }
+    c->groups_valid = ok;
 }
 // A call that completed leaves the hull records and count slots of its jobs reset.
 void end_call(sqd_core* c) { c->clean = c->ny; }
@@ -944,8 +969,8 @@ void drain_criticals(sqd_core* c, unsigned long long k, unsigned long long n_fin
             for(unsigned g = 0; g < src.segs; ++g)
                 ranges.push_back({g * src.seg_cap, std::min(n[static_cast<std::size_t>(g) * dev::kSegStride], src.seg_cap)});
         }
-        // a part's children must fit the critical list and, on a prefiltered or
-        // grouped last level, the undecided list; without static levels a part
+        // a part's children must fit the critical list and, on a prefiltered last
+        // level, the undecided list; without static levels a part
         // is at most a round's final list
         const unsigned long long subs = S > 0 ? c->st_subs[static_cast<std::size_t>(S - 1)] : 1ull;
         const unsigned long long room = c->undec_cap ? std::min(cap, c->undec_cap) : cap;
@@ -1138,14 +1163,13 @@ void configure_core(sqd_core* c, int device, const sqd_program* program, const s
     }
     kmax = std::min(kmax, room / worst_static);
     kmax = std::min(kmax, room / worst_split);
-    // the FP32 prefilter and the binary64 group test list the children they
-    // leave undecided (8 bytes each, level_bytes of them), up to all children
-    // of the level, so a round is bounded by the largest such level's children
-    // per dynamic cuboid
+    // the FP32 prefilter lists the children it leaves undecided (8 bytes each,
+    // level_bytes of them), up to all children of the level, so a round is bounded
+    // by the largest such level's children per dynamic cuboid
     const unsigned long long undec_cap = std::max<unsigned long long>(1024, s.level_bytes / 8);
     unsigned long long worst_undec = 1;
     for(std::size_t L = 0; L < c->st_subs.size() && L < 32; ++L)
-        if(((s.group_levels | s.fp32_prefilter) >> L) & 1u)
+        if((s.fp32_prefilter >> L) & 1u)
             worst_undec = std::max<unsigned long long>(worst_undec, product(c->st_subs, L + 1));
     kmax = std::min(kmax, undec_cap / worst_undec);
     if(kmax == 0) throw Failure(SQD_ERR_CAPACITY, "level buffers too small for one cuboid");
@@ -1172,7 +1196,7 @@ void configure_core(sqd_core* c, int device, const sqd_program* program, const s
     c->scratch.lay(lay, c->N, std::max<unsigned long long>(kmax, 1024), true, false);
     lay.take(c->d_hull, static_cast<std::size_t>(kmax) * c->N * 4);
     lay.take(c->d_range, 3);   // first, last, start flag
-    if(c->fp32 || (s.group_levels & used)) {
+    if(c->fp32) {
         c->undec_cap = undec_cap;
         lay.take(c->d_undec, static_cast<std::size_t>(undec_cap));
     }
@@ -1422,6 +1446,7 @@ int sqd_nonfinal(sqd_core* c, const double* lb, const double* ub, size_t n,
         if(!c || (n && (!lb || !ub || !hull_lb || !hull_ub || !has_hull))) throw std::invalid_argument("null argument");
         hip_check(hipSetDevice(c->device), "hipSetDevice");
         begin_call(c);
+        check_groups_valid(c, lb, ub, n);
         reset_state(c);
         std::vector<double> clb, cub, hlb, hub;
         for(std::size_t off = 0; off < n; off += c->k_max) {
@@ -1464,6 +1489,7 @@ int sqd_final(sqd_core* c, const double* lb, const double* ub, size_t n,
         hip_check(hipSetDevice(c->device), "hipSetDevice");
         if(n > c->fin.cap) throw Failure(SQD_ERR_CAPACITY, "too many boxes for one final pass");
         begin_call(c);
+        check_groups_valid(c, lb, ub, n);
         reset_state(c);
         upload_soa(c, c->fin, lb, ub, n, 0);
         if(c->ks->NSTAT > 0) run_static(c, dev::FINAL, c->fin.view(), nullptr, c->fin.count, n, c->crit.view());

@@ -291,6 +291,9 @@ struct sqd_service {
     uint64_t frontier_in_flight = 0;
     std::map<const sqd_program*, double> frontier_per_unit;
     sqd_service_stats stats{};
+    // how long a batch without jobs stays open, and the workers waiting for memory
+    static constexpr std::chrono::milliseconds kBatchOpen{20};
+    unsigned room_wanted = 0;
     bool stop = false;
     std::vector<std::thread> workers;
 
@@ -342,7 +345,12 @@ struct sqd_service {
                     freed = true;
                     break;
                 }
-            if(!freed) cv.wait(lk);
+            if(!freed) {
+                ++room_wanted;
+                cv.notify_all();   // open batches without jobs give up their cores
+                cv.wait(lk);
+                --room_wanted;
+            }
         }
     }
 
@@ -504,8 +512,9 @@ struct sqd_service {
             std::vector<uint64_t> row_cuboids(rows, 0);
             const uint64_t bpc = cuboid_bytes(prog);
             uint32_t running = 0;
+            bool kept_open = false;
             auto admit = [&] {   // with the lock held: queued jobs of prog into free rows
-                const bool joining = running > 0;
+                const bool joining = running > 0 || kept_open;
                 for(uint32_t r = 0; r < rows; ++r) {
                     if(row_job[r]) continue;
                     const uint64_t next = peek_queued(prog);
@@ -530,7 +539,18 @@ struct sqd_service {
             };
             admit();
             std::vector<sqd_job_counts> jc(rows);
-            while(running > 0) {
+            // The batch stays open for a moment after its last job, as long as
+            // nothing else is queued and no worker waits for memory, so that the
+            // next job of the program joins it on this core instead of opening
+            // another one.
+            auto keep_open = [&] {
+                if(running > 0) return true;
+                kept_open = cv.wait_for(lk, kBatchOpen, [&] { return stop || !queue.empty() || room_wanted > 0; }) &&
+                            !stop && room_wanted == 0;
+                if(kept_open) admit();
+                return running > 0;
+            };
+            while(keep_open()) {
                 lk.unlock();
                 uint64_t finished = 0;
                 uint32_t active = 0;

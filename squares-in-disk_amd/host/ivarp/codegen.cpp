@@ -255,7 +255,7 @@ struct Emitter {
                 // domain checks only where the compile-time bounds leave [-1, 1]
                 const bool chk_lb = KN(0).lb < fpb::int_to_fp(-1), chk_ub = KN(0).ub > fpb::int_to_fp(1);
                 o << "const IV " << v(id) << " = iv_acos<" << (chk_lb ? "true" : "false") << ", "
-                  << (chk_ub ? "true" : "false") << ">(" << v(K(0)) << ");";
+                  << (chk_ub ? "true" : "false") << ", EXACT>(" << v(K(0)) << ");";
                 break;
             }
             case FOp::BoolConst: o << "const IB " << b(id) << "{" << (n.b_def ? "true" : "false") << ", " << (n.b_poss ? "true" : "false") << "};"; break;
@@ -282,11 +282,29 @@ std::string generate(const flat::Program& p, const std::string& key) {
     for(std::size_t i = 0; i < p.splits.size(); ++i) (p.splits[i].dynamic ? dyn : sta).push_back(static_cast<int>(i));
     std::ostringstream body;
 
-    // constraint predicates, one function per constraint root
+    // Constraint predicates, one function per constraint root.  EXACT selects the
+    // correctly rounded arc cosines of the reference; with EXACT = false they are
+    // the cheap enclosures (some 40 operations instead of thousands), whose
+    // intervals contain the exact ones: a constraint that fails with them fails
+    // exactly too, so the checks below try it first.
+    std::vector<char> acos_dep(p.nodes.size(), 0);   // nodes that read an arc cosine
+    for(std::size_t i = 0; i < p.nodes.size(); ++i) {
+        acos_dep[i] = p.nodes[i].op == FOp::Acos;
+        for(int k : p.nodes[i].kids) acos_dep[i] = acos_dep[i] || acos_dep[static_cast<std::size_t>(k)];
+    }
+    // the checks `if(!c(...).poss) <fail>` of a list of constraints: all with
+    // enclosures, then those that read an arc cosine again with the exact values
+    // (in binary32 the enclosures are all there is)
+    auto checks = [&](std::ostringstream& o, const std::vector<int>& list, const std::string& indent, const std::string& fail) {
+        for(int c : list) o << indent << "if(!c" << c << "<false>(lb, ub, C).poss) " << fail << "\n";
+        for(int c : list)
+            if(acos_dep[static_cast<std::size_t>(c)])
+                o << indent << "if(sizeof(Num) == sizeof(double) && !c" << c << "<true>(lb, ub, C).poss) " << fail << "\n";
+    };
     std::map<int, bool> roots;
     for(const auto& r : p.rows) for(int c : r) roots[c] = true;
     for(const auto& kv : roots) {
-        body << "    template<class Num> __device__ __forceinline__ static IB c" << kv.first
+        body << "    template<bool EXACT, class Num> __device__ __forceinline__ static IB c" << kv.first
              << "(const Num (&lb)[N], const Num (&ub)[N], const Num* C) {\n";
         body << "        using IV = IVT<Num>;\n        (void)lb; (void)ub; (void)C;\n";
         body << e.eval(kv.first, "        ");
@@ -301,7 +319,7 @@ std::string generate(const flat::Program& p, const std::string& key) {
         const bool cmp = n.op == FOp::Lt || n.op == FOp::Le || n.op == FOp::Gt || n.op == FOp::Ge;
         body << "    template<class Num> __device__ static IVT<Num> d" << c
              << "(const Num (&lb)[N], const Num (&ub)[N], const Num* C) {\n";
-        body << "        using IV = IVT<Num>;\n        (void)lb; (void)ub; (void)C;\n";
+        body << "        using IV = IVT<Num>;\n        constexpr bool EXACT = true;\n        (void)lb; (void)ub; (void)C; (void)EXACT;\n";
         if(cmp) {
             body << e.eval(c, "        ");
             body << "        (void)" << e.b(c) << ";\n";
@@ -322,7 +340,7 @@ std::string generate(const flat::Program& p, const std::string& key) {
     // the IBool of constraint j (in cons_id order) on a box, evaluated exactly as
     // apply and the row checks evaluate them
     body << "    template<class Num> __device__ static IVT<Num> bound_value(int k, const Num (&lb)[N], const Num (&ub)[N], const Num* C) {\n";
-    body << "        using IV = IVT<Num>;\n        (void)lb; (void)ub; (void)C;\n        switch(k) {\n";
+    body << "        using IV = IVT<Num>;\n        constexpr bool EXACT = true;\n        (void)lb; (void)ub; (void)C; (void)EXACT;\n        switch(k) {\n";
     for(std::size_t k = 0; k < p.bounds.size(); ++k) {
         body << "        case " << k << ": {\n" << e.eval(p.bounds[k].expr, "            ");
         body << "            return " << e.v(p.bounds[k].expr) << ";\n        }\n";
@@ -330,11 +348,11 @@ std::string generate(const flat::Program& p, const std::string& key) {
     body << "        default: return IV{Num(1), Num(0), true};\n        }\n    }\n";
     body << "    template<class Num> __device__ static IB cons_value(int j, const Num (&lb)[N], const Num (&ub)[N], const Num* C) {\n";
     body << "        switch(j) {\n";
-    for(std::size_t j = 0; j < cons.size(); ++j) body << "        case " << j << ": return c" << cons[j] << "(lb, ub, C);\n";
+    for(std::size_t j = 0; j < cons.size(); ++j) body << "        case " << j << ": return c" << cons[j] << "<true>(lb, ub, C);\n";
     body << "        default: return IB{false, true};\n        }\n    }\n";
     // bound application
     body << "    template<class Num> __device__ __forceinline__ static int apply(int k, Num (&lb)[N], Num (&ub)[N], const Num* C) {\n";
-    body << "        using IV = IVT<Num>;\n        (void)lb; (void)ub; (void)C;\n        switch(k) {\n";
+    body << "        using IV = IVT<Num>;\n        constexpr bool EXACT = true;\n        (void)lb; (void)ub; (void)C; (void)EXACT;\n        switch(k) {\n";
     for(std::size_t k = 0; k < p.bounds.size(); ++k) {
         const flat::FBound& bd = p.bounds[k];
         const int t = bd.target;
@@ -387,28 +405,29 @@ std::string generate(const flat::Program& p, const std::string& key) {
         for(int r = from; r < to; ++r)
             for(int c : p.rows[static_cast<std::size_t>(r)]) level.push_back(c);
         body << "        if constexpr(L == " << L << ") {\n";
-        for(int c : level) body << "            if(!c" << c << "(lb, ub, C).poss) return true;\n";
+        checks(body, level, "            ", "return true;");
         body << "        }\n";
     }
     body << "        return false;\n    }\n";
     body << "    template<class Num> __device__ __forceinline__ static bool all_satisfied(const Num (&lb)[N], const Num (&ub)[N], const Num* C) {\n";
-    for(int c : p.rows[static_cast<std::size_t>(p.nargs - 1)]) body << "        if(!c" << c << "(lb, ub, C).poss) return false;\n";
+    checks(body, p.rows[static_cast<std::size_t>(p.nargs - 1)], "        ", "return false;");
     body << "        (void)lb; (void)ub; (void)C;\n        return true;\n    }\n";
 
-    // Hoisted row checks for the FP32 prefilter.  At static level L the rows
+    // Hoisted row checks for the FP32 prefilter and the group tests (arc cosines
+    // as enclosures: what passes is decided by rows_violated).  At static level L the rows
     // are checked on a box whose variables other than the split variable A are
     // the parent's for every child, so each term free of A has the same value
     // for all children of a parent: hoist<L> computes the terms the other terms
     // read (the frontier) once per parent into Hoist<L>, and
     // rows_violated_hoisted<L> evaluates the rest per child, with the same
-    // results as rows_violated<L> on that box.
+    // results as rows_violated<L>'s first checks on that box.
     std::ostringstream hoist_types, hoist_fns;
     hoist_fns << "    template<int L, class Num> __device__ __forceinline__ static void hoist(const Num (&lb)[N], const Num (&ub)[N], "
-                 "const Num* C, Hoist<L, Num>& h) {\n        using IV = IVT<Num>;\n        (void)lb; (void)ub; (void)C; (void)h;\n";
+                 "const Num* C, Hoist<L, Num>& h) {\n        using IV = IVT<Num>;\n        constexpr bool EXACT = false;\n        (void)lb; (void)ub; (void)C; (void)h; (void)EXACT;\n";
     std::ostringstream rows_h;
     rows_h << "    template<int L, class Num> __device__ __forceinline__ static bool rows_violated_hoisted(const Num (&lb)[N], "
               "const Num (&ub)[N], const Num* C, const Hoist<L, Num>& h) {\n        using IV = IVT<Num>;\n"
-              "        (void)lb; (void)ub; (void)C; (void)h;\n";
+              "        constexpr bool EXACT = false;\n        (void)lb; (void)ub; (void)C; (void)h; (void)EXACT;\n";
     std::string hoist_sel = "NoHoist";
     for(std::size_t L = sta.size(); L-- > 0;) {
         const int A = p.splits[static_cast<std::size_t>(sta[L])].arg;
@@ -519,13 +538,14 @@ std::string generate(const flat::Program& p, const std::string& key) {
     table("dyn_subs", dyn, [](const flat::FSplit& s) { return static_cast<int>(s.subs); });
     table("st_arg", sta, [](const flat::FSplit& s) { return s.arg; });
     table("st_subs", sta, [](const flat::FSplit& s) { return static_cast<int>(s.subs); });
-    // Register budget of the binary64 static level kernels as resident waves
-    // per SIMD (0: the compiler's choice), measured per kernel (per proof, with
-    // the constraint functions inlined): One's and Two's level 1 at 4 (128
-    // VGPRs, a few spilled; 3 was slower), Three's level 1 at 4 (274 against
-    // 292 us), More1's level 1 at 3 (264 against 301 ms at the compiler's 176
-    // VGPRs), Four's level 2 at 3 (3.46 against 3.92 ms) and More2's level 2 at
-    // 3 (19.8 ms; 4 spilled 426 VGPRs and took 38.7 ms).
+    // Register budget of the per-child binary64 level kernels (k_static_level) as
+    // resident waves per SIMD (0: the compiler's choice).  On a last level that is
+    // the pass over the children binary32 left undecided; the values were measured
+    // on whole levels decided child by child: One's and Two's level 1 at 4 (128
+    // VGPRs, a few spilled; 3 was slower), Three's level 1 at 4 (274 against 292
+    // us), More1's level 1 at 3 (264 against 301 ms at the compiler's 176 VGPRs),
+    // Four's level 2 at 3 (3.46 against 3.92 ms) and More2's level 2 at 3 (19.8 ms;
+    // 4 spilled 426 VGPRs and took 38.7 ms).
     int waves_l1 = 0, waves_l2 = 0;
     if(key == "one" || key == "two" || key == "three") waves_l1 = 4;
     if(key == "more1") waves_l1 = 3;
