@@ -68,8 +68,10 @@ typedef struct sqd_settings {
                                       0 = off, SQD_FP32_ALL_LEVELS = every level (no
                                       counterpart in the reference, which evaluates
                                       everything in binary64) */
-    uint32_t graphs;               /* nonzero: sqd_prove replays its rounds as captured HIP
-                                      graphs from the second proof on a core (default 1) */
+    uint32_t graphs;               /* nonzero: rounds that are enqueued whole (continuous batches;
+                                      proofs with a critical sink or progress reports) are
+                                      replayed as captured HIP graphs from the second proof on a
+                                      core (default 1) */
     uint32_t prefilter_group;      /* FP32 prefilter: consecutive children of one parent a
                                       lane first tests as one group (a power of two up to
                                       64; 0 = chosen per launch, 1 = no groups) */

@@ -98,6 +98,31 @@ struct BoxList {
 constexpr unsigned kSegs = 16;
 constexpr unsigned kSegStride = 32;   // 64-bit words from one segment's counter to the next
 
+// What the first kernel of a round writes when it takes the round's cuboids from
+// the frontier itself (LevelArgs::pop): pop_round() below.
+struct RoundWords {
+    unsigned long long round_k, round_base;   // the round pops [round_base, round_base + round_k)
+    unsigned long long frontier_full;         // nonzero: a round could not pop anything
+    unsigned long long frontier_peak;         // most cuboids the frontier held after a round
+    unsigned long long rounds;                // rounds begun
+    unsigned long long fin_count, spl_count;  // the round's hulls to finish and to split
+};
+// Start of a proof, done by the first kernel of the initial queue (one block per
+// job): n_words words at `words` (the control block) and the counters of the
+// segmented lists to zero, the job's range from host memory to `range`, and the
+// box (N lb, N ub) as the level's only input.  With `flagged` only the jobs whose
+// start flag is set start; the others get no input.
+struct StartArgs {
+    unsigned long long* words;        // nullptr: no start (the input list is used)
+    unsigned n_words;
+    const double* box;
+    const unsigned* host_ranges;      // pinned: lo[64], hi[64], start[64]
+    unsigned long long* range;        // first, last, start flag
+    unsigned flagged;
+    unsigned long long* seg_counters;
+    unsigned seg_lists;
+};
+
 // Arguments of a level kernel.  The input range lives in device memory (the
 // round's pop position and size, or a list's counter), so a whole round can be
 // enqueued without the host knowing its size.
@@ -125,6 +150,10 @@ struct LevelArgs {
     // `jobs` is the number of rows the host launches
     unsigned long long job_stride;
     unsigned jobs;
+    // first level of a round: `in` is the frontier, of which the round takes the
+    // top min(k_max, n, room for the children) cuboids (nullptr: in_base, in_count)
+    RoundWords* pop;
+    unsigned long long pop_max, pop_fanout;
 };
 
 // ---------------------------------------------------------------- batched jobs
@@ -162,6 +191,7 @@ __device__ __forceinline__ LevelArgs job_args(LevelArgs a) {
     a.undec = job_ptr(a.undec, off);
     a.undec_count = job_ptr(a.undec_count, off);
     a.init_range = job_ptr(a.init_range, off);
+    a.pop = job_ptr(a.pop, off);
     return a;
 }
 
@@ -414,13 +444,36 @@ struct Inputs {
 template<int SHIFT> __device__ __forceinline__ unsigned row_add(unsigned v) {
     return v + static_cast<unsigned>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x110 + SHIFT, 0xf, 0xf, false));
 }
+// A round takes K = min(k_max, n, room / (fanout - 1)) cuboids from the top of a
+// frontier of n; their places are reused by the children the round pushes.
+__device__ __forceinline__ unsigned long long pop_size(unsigned long long n, unsigned long long k_max,
+                                                       unsigned long long cap, unsigned long long fanout) {
+    unsigned long long k = n < k_max ? n : k_max;
+    if(fanout > 1) {
+        const unsigned long long lim = (cap > n ? cap - n : 0ull) / (fanout - 1);
+        k = k < lim ? k : lim;
+    }
+    return k;
+}
+// The round's record (by one thread): it is read from the next kernel on.  The
+// frontier's count itself is lowered by k_hull_finalize, when no block of the
+// first level reads it any more.
+__device__ __forceinline__ void pop_round(RoundWords& r, unsigned long long n, unsigned long long k) {
+    if(k == 0 && n > 0) r.frontier_full = 1ull;
+    if(r.rounds > 0 && n > r.frontier_peak) r.frontier_peak = n;   // n: after the round before
+    ++r.rounds;
+    r.round_k = k;
+    r.round_base = n - k;
+    r.fin_count = 0ull;
+    r.spl_count = 0ull;
+}
 // Called by every thread of the block.
 template<bool SEG>
 __device__ __forceinline__ Inputs<SEG> level_inputs(const LevelArgs& a) {
     Inputs<SEG> in;
     in.seg_cap = a.in.seg_cap;
-    in.base = a.in_base ? *a.in_base : 0ull;
     in.dense = true;
+    in.base = 0;
     in.before = 0;
     in.table = nullptr;
     if constexpr(SEG) {
@@ -444,7 +497,17 @@ __device__ __forceinline__ Inputs<SEG> level_inputs(const LevelArgs& a) {
             return in;
         }
     }
+    if constexpr(!SEG) {
+        if(a.pop) {
+            const unsigned long long n = *a.in.count;
+            in.n = pop_size(n, a.pop_max, a.in.cap, a.pop_fanout);
+            in.base = n - in.n;
+            if(blockIdx.x == 0 && threadIdx.x == 0) pop_round(*a.pop, n, in.n);
+            return in;
+        }
+    }
     const unsigned long long n = *a.in_count;
+    in.base = a.in_base ? *a.in_base : 0ull;
     const unsigned long long room = a.in.cap > in.base ? a.in.cap - in.base : 0ull;
     in.n = n < room ? n : room;
     return in;
@@ -1015,7 +1078,7 @@ void k_static_grouped(LevelArgs job0) {
 // initial queue).  The last level keeps children that possibly satisfy every
 // constraint and appends them to the output (the cuboid stack).
 template<class P, int MODE, int J>
-__global__ __launch_bounds__(kBlock) SQD_LEVEL_ATTR void k_dynamic_level(LevelArgs job0) {
+__global__ __launch_bounds__(kBlock) SQD_LEVEL_ATTR void k_dynamic_level(LevelArgs job0, StartArgs start) {
     const LevelArgs args = job_args(job0);
     constexpr int N = P::N;
     constexpr int ARG = P::dyn_arg(J);
@@ -1025,12 +1088,43 @@ __global__ __launch_bounds__(kBlock) SQD_LEVEL_ATTR void k_dynamic_level(LevelAr
     const double* const s_c = nullptr;   // constants are literals in the generated code (P::kc)
     __shared__ PropScratch<P> s_prop;
     enter_round_down();
-    const Inputs<(J > 0)> in = level_inputs<(J > 0)>(args);
-    const unsigned long long n_items = in.n;
     // the initial queue may start from a range of the first variable's subdivisions
     constexpr bool RANGED = (MODE == INIT && J == 0);
-    const unsigned long long r_lo = RANGED && args.init_range ? args.init_range[0] : 0ull;
-    const unsigned long long r_n = RANGED && args.init_range ? args.init_range[1] - r_lo : static_cast<unsigned long long>(SUBS);
+    Inputs<(J > 0)> in;
+    unsigned long long r_lo = 0ull, r_n = static_cast<unsigned long long>(SUBS);
+    bool from_box = false;
+    if constexpr(RANGED) {
+        from_box = start.words != nullptr;
+        if(from_box) {
+            const unsigned long long off = job_offset(args.job_stride);
+            const unsigned lo = start.host_ranges[blockIdx.y], hi = start.host_ranges[64 + blockIdx.y];
+            if(start.flagged && !start.host_ranges[128 + blockIdx.y]) return;   // the whole row
+            unsigned long long* words = job_ptr(start.words, off);
+            // (device-scope stores: the block's atomics below meet them)
+            for(unsigned i = threadIdx.x; i < start.n_words; i += blockDim.x)
+                __hip_atomic_store(words + i, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            unsigned long long* segs = job_ptr(start.seg_counters, off);
+            for(unsigned i = threadIdx.x; i < start.seg_lists * kSegs; i += blockDim.x)
+                __hip_atomic_store(segs + i * kSegStride, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __syncthreads();
+            r_lo = lo;
+            r_n = hi - lo;
+            in.dense = true;
+            in.base = 0ull;
+            in.n = 1ull;
+            in.seg_cap = 0ull;
+            in.before = 0u;
+            in.table = nullptr;
+        }
+    }
+    if(!from_box) {
+        in = level_inputs<(J > 0)>(args);
+        if(RANGED && args.init_range) {
+            r_lo = args.init_range[0];
+            r_n = args.init_range[1] - r_lo;
+        }
+    }
+    const unsigned long long n_items = in.n;
     const unsigned long long total = n_items * r_n;
     const unsigned long long stride = static_cast<unsigned long long>(gridDim.x) * blockDim.x;
     const unsigned long long first = static_cast<unsigned long long>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -1045,8 +1139,14 @@ __global__ __launch_bounds__(kBlock) SQD_LEVEL_ATTR void k_dynamic_level(LevelAr
         const unsigned long long src = in.entry(w / r_n, w < total);
         if(w < total) {
             const int i = static_cast<int>(r_lo + w % r_n);
-            load_box<P>(args.in, src, lb, ub);
-            depth = args.in.depth ? args.in.depth[src] : 0u;
+            if(from_box) {
+                const double* box = job_ptr(start.box, job_offset(args.job_stride));
+#pragma unroll
+                for(int a = 0; a < N; ++a) { lb[a] = box[a]; ub[a] = box[N + a]; }
+            } else {
+                load_box<P>(args.in, src, lb, ub);
+                depth = args.in.depth ? args.in.depth[src] : 0u;
+            }
             ++c_cub;
             const double pl = lb[ARG], pu = ub[ARG];
             const double wd = split_width(pl, pu, SUBS);
@@ -1075,9 +1175,6 @@ __global__ __launch_bounds__(kBlock) SQD_LEVEL_ATTR void k_dynamic_level(LevelAr
 }
 
 // ---------------------------------------------------------------- round glue
-// Turn the hull records of one round into boxes.  Hulls at depth >= generations
-// go to `fin` (final pass), the others to `spl` with depth + 1 (dynamic split).
-// Without static variables the popped cuboid itself is the only leaf.
 // Hull records start as (min key, max key, zero-sign keys) = (~0, 0, ~0, ~0)
 // and are put back to that state by the kernel that consumes them.
 __device__ __forceinline__ void clear_hull_record(unsigned long long* rec, int n_args) {
@@ -1091,15 +1188,13 @@ __device__ __forceinline__ void clear_hull_record(unsigned long long* rec, int n
 
 // Turn the hull records of one round into boxes.  Hulls at depth >= generations
 // go to `fin` (final pass), the others to `spl` with depth + 1 (dynamic split).
-// Without static variables the popped cuboid itself is the only leaf.  The
-// round's items are [*base, *base + *count) of `items`.  Row blockIdx.y of the
-// grid works on job blockIdx.y.
+// The round's items are [*base, *base + *count) of `items`.  Row blockIdx.y of
+// the grid works on job blockIdx.y.
 template<class P>
 __global__ __launch_bounds__(kBlock) void k_hull_finalize(BoxList items, const unsigned long long* base_ptr,
                                                           const unsigned long long* count_ptr, unsigned long long* hull,
                                                           BoxList fin, BoxList spl, DeviceCounters* counters,
-                                                          unsigned long long* block_counts, unsigned generations,
-                                                          unsigned long long job_stride) {
+                                                          unsigned generations, unsigned long long job_stride) {
     constexpr int N = P::N;
     const unsigned long long off = job_offset(job_stride);
     items = job_list(items, off);
@@ -1109,33 +1204,28 @@ __global__ __launch_bounds__(kBlock) void k_hull_finalize(BoxList items, const u
     count_ptr = job_ptr(count_ptr, off);
     hull = job_ptr(hull, off);
     counters = job_ptr(counters, off);
-    block_counts = job_ptr(block_counts, off);
     const unsigned long long n = *count_ptr, base = *base_ptr;
     const unsigned long long d = static_cast<unsigned long long>(blockIdx.x) * blockDim.x + threadIdx.x;
+    // the round's cuboids leave the frontier
+    if(blockIdx.x == 0 && threadIdx.x == 0) *items.count = base;
     bool have = false;
     double lb[N], ub[N];
     unsigned depth = 0;
     if(d < n) {
         depth = items.depth[base + d];
-        if(P::NSTAT == 0) {
-            load_box<P>(items, base + d, lb, ub);
-            have = true;
-        } else {
-            unsigned long long* rec = hull + d * N * 4;
-            have = rec[0] != ~0ull;
-            if(have) {
+        unsigned long long* rec = hull + d * N * 4;
+        have = rec[0] != ~0ull;
+        if(have) {
 #pragma unroll
-                for(int a = 0; a < N; ++a) {
-                    lb[a] = from_order_key(rec[a * 4 + 0]);
-                    ub[a] = from_order_key(rec[a * 4 + 1]);
-                    if(lb[a] == 0.0) lb[a] = (rec[a * 4 + 2] & 1ull) ? -0.0 : 0.0;
-                    if(ub[a] == 0.0) ub[a] = (rec[a * 4 + 3] & 1ull) ? -0.0 : 0.0;
-                }
-                clear_hull_record(rec, N);
+            for(int a = 0; a < N; ++a) {
+                lb[a] = from_order_key(rec[a * 4 + 0]);
+                ub[a] = from_order_key(rec[a * 4 + 1]);
+                if(lb[a] == 0.0) lb[a] = (rec[a * 4 + 2] & 1ull) ? -0.0 : 0.0;
+                if(ub[a] == 0.0) ub[a] = (rec[a * 4 + 3] & 1ull) ? -0.0 : 0.0;
             }
+            clear_hull_record(rec, N);
         }
     }
-    if(P::NSTAT == 0) block_counts_add(block_counts, 0ull, have ? 1ull : 0ull, 0ull);
     const bool to_final = have && depth >= generations;
     const bool to_split = have && !to_final;
     const unsigned long long pf = wave_append(to_final, fin.count);
@@ -1148,6 +1238,74 @@ __global__ __launch_bounds__(kBlock) void k_hull_finalize(BoxList items, const u
         if(ps < spl.cap) { store_box<P>(spl, ps, lb, ub); spl.depth[ps] = depth + 1; }
         else atomicAdd(&counters->overflow, 1ull);
     }
+}
+
+// A round up to its dynamic split without static variables, one block per job:
+// the round's cuboids are taken from the frontier; each is its own only leaf and
+// hull and goes to `spl` with depth + 1 or, at the last generation, to `fin` and
+// to the criticals.  (Three kernels before, 4 to 5 us each for a few cuboids.)
+template<class P>
+__global__ __launch_bounds__(kBlock) void k_round_nostatic(BoxList stack, RoundWords* round, unsigned long long k_max,
+                                                           unsigned long long fanout, BoxList fin, BoxList spl,
+                                                           BoxList crit, DeviceCounters* counters,
+                                                           unsigned long long* block_counts, unsigned generations,
+                                                           unsigned long long job_stride) {
+    constexpr int N = P::N;
+    const unsigned long long off = job_offset(job_stride);
+    stack = job_list(stack, off);
+    fin = job_list(fin, off);
+    spl = job_list(spl, off);
+    crit = job_list(crit, off);
+    round = job_ptr(round, off);
+    counters = job_ptr(counters, off);
+    block_counts = job_ptr(block_counts, off);
+    const unsigned long long had = *stack.count;
+    const unsigned long long n = pop_size(had, k_max, stack.cap, fanout), base = had - n;
+    __shared__ unsigned long long s_fin, s_spl, s_crit;
+    __syncthreads();   // every wave has read the count
+    if(threadIdx.x == 0) {
+        pop_round(*round, had, n);
+        *stack.count = base;
+        s_fin = 0ull;
+        s_spl = 0ull;
+        s_crit = *crit.count;
+    }
+    __syncthreads();
+    unsigned long long c_leaf = 0, c_crit = 0;
+    for(unsigned long long d0 = 0; d0 < n; d0 += kBlock) {
+        const unsigned long long d = d0 + threadIdx.x;
+        const bool have = d < n;
+        double lb[N], ub[N];
+        unsigned depth = 0;
+        if(have) {
+            depth = stack.depth[base + d];
+            load_box<P>(stack, base + d, lb, ub);
+            ++c_leaf;
+        }
+        const bool to_final = have && depth >= generations;
+        const bool to_split = have && !to_final;
+        const unsigned long long pf = wave_append(to_final, &s_fin);
+        const unsigned long long pc = wave_append(to_final, &s_crit);
+        const unsigned long long ps = wave_append(to_split, &s_spl);
+        if(to_final) {
+            ++c_leaf;
+            ++c_crit;
+            if(pf < fin.cap) { store_box<P>(fin, pf, lb, ub); fin.depth[pf] = depth; }
+            else atomicAdd(&counters->overflow, 1ull);
+            if(pc < crit.cap) store_box<P>(crit, pc, lb, ub);
+        }
+        if(to_split) {
+            if(ps < spl.cap) { store_box<P>(spl, ps, lb, ub); spl.depth[ps] = depth + 1; }
+            else atomicAdd(&counters->overflow, 1ull);
+        }
+    }
+    __syncthreads();
+    if(threadIdx.x == 0) {
+        *fin.count = s_fin;
+        *spl.count = s_spl;
+        *crit.count = s_crit;
+    }
+    block_counts_add(block_counts, 0ull, c_leaf, c_crit);
 }
 
 // Decode hull records in input order (sqd_nonfinal): entry d of `out` holds the
@@ -1179,7 +1337,7 @@ __global__ __launch_bounds__(kBlock) void k_hull_decode(BoxList items, unsigned 
     has[d] = ok ? 1 : 0;
 }
 
-// Final pass without static variables: every cuboid is one critical leaf.  Row
+// Final pass without static variables outside a round: every cuboid is one critical leaf.  Row
 // blockIdx.y of the grid works on job blockIdx.y.
 template<class P>
 __global__ __launch_bounds__(kBlock) void k_final_nostatic(BoxList fin, BoxList out, unsigned long long* block_counts,

@@ -23,16 +23,23 @@ struct KernelSet {
     // dev::kModeGroup the binary64 group test.
     hipError_t (*static_level)(int mode, int level, const dev::LevelArgs& a, unsigned long long max_children,
                                unsigned cus, unsigned grid, hipStream_t s);
-    hipError_t (*dynamic_level)(int mode, int level, const dev::LevelArgs& a, unsigned long long max_children,
-                                unsigned cus, unsigned grid, hipStream_t s);
+    // `start` (words != nullptr) makes the initial queue's first level the start of
+    // the proof; its children must fit one block.
+    hipError_t (*dynamic_level)(int mode, int level, const dev::LevelArgs& a, const dev::StartArgs& start,
+                                unsigned long long max_children, unsigned cus, unsigned grid, hipStream_t s);
     // Hulls of the round's items [*base, *base + *count) (at most max_n of them).
     // These three launch `jobs` grid rows, row j on job j's memory (job 0's
     // pointers plus j * job_stride bytes); the level launches take the same from
     // LevelArgs.
     hipError_t (*hull_finalize)(dev::BoxList items, const unsigned long long* base, const unsigned long long* count,
                                 unsigned long long max_n, unsigned long long* hull, dev::BoxList fin,
-                                dev::BoxList spl, dev::DeviceCounters* c, unsigned long long* block_counts,
-                                unsigned gens, unsigned jobs, unsigned long long job_stride, hipStream_t s);
+                                dev::BoxList spl, dev::DeviceCounters* c, unsigned gens, unsigned jobs,
+                                unsigned long long job_stride, hipStream_t s);
+    // A round up to its split for programs without static levels (k_round_nostatic).
+    hipError_t (*round_nostatic)(dev::BoxList stack, dev::RoundWords* round, unsigned long long k_max,
+                                 unsigned long long fanout, dev::BoxList fin, dev::BoxList spl, dev::BoxList crit,
+                                 dev::DeviceCounters* c, unsigned long long* block_counts, unsigned gens, unsigned jobs,
+                                 unsigned long long job_stride, hipStream_t s);
     hipError_t (*final_nostatic)(dev::BoxList fin, dev::BoxList out, unsigned long long* block_counts, unsigned grid,
                                  unsigned jobs, unsigned long long job_stride, hipStream_t s);
     hipError_t (*initial_box)(const double* lb, const double* ub, const double* consts, double* out,
@@ -108,9 +115,11 @@ hipError_t launch_one_static(const dev::LevelArgs& a, unsigned long long max_chi
         if(e != hipSuccess) return e;
     }
     if constexpr(F32 || L != P::NSTAT - 1) {
+        dev::LevelArgs b = a;
+        if(F32) b.pop = nullptr;   // the prefilter took the round's cuboids
         static const unsigned per_cu = blocks_per_cu(dev::k_static_level<P, MODE, L, F32>);
         hipLaunchKernelGGL((dev::k_static_level<P, MODE, L, F32>),
-                           dim3(level_grid(per_cu, cus, jobs_of(a), max_children, grid), jobs_of(a)), dim3(dev::kBlock), 0, s, a);
+                           dim3(level_grid(per_cu, cus, jobs_of(a), max_children, grid), jobs_of(a)), dim3(dev::kBlock), 0, s, b);
     }
     return hipGetLastError();
 }
@@ -123,11 +132,12 @@ hipError_t launch_grouped(int level, const dev::LevelArgs& a, unsigned long long
     return e;
 }
 template<class P, int MODE, int J>
-hipError_t launch_one_dynamic(const dev::LevelArgs& a, unsigned long long max_children, unsigned cus, unsigned grid,
-                              hipStream_t s) {
+hipError_t launch_one_dynamic(const dev::LevelArgs& a, const dev::StartArgs& start, unsigned long long max_children,
+                              unsigned cus, unsigned grid, hipStream_t s) {
     static const unsigned per_cu = blocks_per_cu(dev::k_dynamic_level<P, MODE, J>);
     hipLaunchKernelGGL((dev::k_dynamic_level<P, MODE, J>),
-                       dim3(level_grid(per_cu, cus, jobs_of(a), max_children, grid), jobs_of(a)), dim3(dev::kBlock), 0, s, a);
+                       dim3(start.words ? 1u : level_grid(per_cu, cus, jobs_of(a), max_children, grid), jobs_of(a)),
+                       dim3(dev::kBlock), 0, s, a, start);
     return hipGetLastError();
 }
 template<class P, int MODE, bool F32, int... L>
@@ -139,11 +149,11 @@ hipError_t launch_static(int level, const dev::LevelArgs& a, unsigned long long 
     return e;
 }
 template<class P, int MODE, int... J>
-hipError_t launch_dynamic(int level, const dev::LevelArgs& a, unsigned long long mc, unsigned cus, unsigned grid,
-                          hipStream_t s, std::integer_sequence<int, J...>) {
+hipError_t launch_dynamic(int level, const dev::LevelArgs& a, const dev::StartArgs& st, unsigned long long mc, unsigned cus,
+                          unsigned grid, hipStream_t s, std::integer_sequence<int, J...>) {
     hipError_t e = hipErrorInvalidValue;
-    (void)a; (void)mc; (void)cus; (void)grid; (void)s; (void)level;
-    ((level == J ? (e = launch_one_dynamic<P, MODE, J>(a, mc, cus, grid, s), 0) : 0), ...);
+    (void)a; (void)st; (void)mc; (void)cus; (void)grid; (void)s; (void)level;
+    ((level == J ? (e = launch_one_dynamic<P, MODE, J>(a, st, mc, cus, grid, s), 0) : 0), ...);
     return e;
 }
 
@@ -161,23 +171,38 @@ hipError_t static_level(int mode, int level, const dev::LevelArgs& a, unsigned l
     return hipErrorInvalidValue;
 }
 template<class P>
-hipError_t dynamic_level(int mode, int level, const dev::LevelArgs& a, unsigned long long mc, unsigned cus,
-                         unsigned grid, hipStream_t s) {
+hipError_t dynamic_level(int mode, int level, const dev::LevelArgs& a, const dev::StartArgs& start, unsigned long long mc,
+                         unsigned cus, unsigned grid, hipStream_t s) {
     auto seq = std::make_integer_sequence<int, P::NDYN>{};
-    if(mode == dev::SPLIT) return launch_dynamic<P, dev::SPLIT>(level, a, mc, cus, grid, s, seq);
-    if(mode == dev::INIT) return launch_dynamic<P, dev::INIT>(level, a, mc, cus, grid, s, seq);
+    if(mode == dev::SPLIT) return launch_dynamic<P, dev::SPLIT>(level, a, start, mc, cus, grid, s, seq);
+    if(mode == dev::INIT) return launch_dynamic<P, dev::INIT>(level, a, start, mc, cus, grid, s, seq);
     return hipErrorInvalidValue;
 }
 template<class P>
 hipError_t hull_finalize(dev::BoxList items, const unsigned long long* base, const unsigned long long* count,
                          unsigned long long max_n, unsigned long long* hull, dev::BoxList fin, dev::BoxList spl,
-                         dev::DeviceCounters* c, unsigned long long* block_counts, unsigned gens, unsigned jobs,
-                         unsigned long long job_stride, hipStream_t s) {
+                         dev::DeviceCounters* c, unsigned gens, unsigned jobs, unsigned long long job_stride,
+                         hipStream_t s) {
     if(max_n == 0) return hipSuccess;
-    unsigned grid = static_cast<unsigned>((max_n + dev::kBlock - 1) / dev::kBlock);
-    hipLaunchKernelGGL((dev::k_hull_finalize<P>), dim3(grid, jobs ? jobs : 1u), dim3(dev::kBlock), 0, s, items, base,
-                       count, hull, fin, spl, c, block_counts, gens, job_stride);
-    return hipGetLastError();
+    if constexpr(P::NSTAT > 0) {
+        unsigned grid = static_cast<unsigned>((max_n + dev::kBlock - 1) / dev::kBlock);
+        hipLaunchKernelGGL((dev::k_hull_finalize<P>), dim3(grid, jobs ? jobs : 1u), dim3(dev::kBlock), 0, s, items, base,
+                           count, hull, fin, spl, c, gens, job_stride);
+        return hipGetLastError();
+    }
+    return hipErrorInvalidValue;
+}
+template<class P>
+hipError_t round_nostatic(dev::BoxList stack, dev::RoundWords* round, unsigned long long k_max, unsigned long long fanout,
+                          dev::BoxList fin, dev::BoxList spl, dev::BoxList crit, dev::DeviceCounters* c,
+                          unsigned long long* block_counts, unsigned gens, unsigned jobs, unsigned long long job_stride,
+                          hipStream_t s) {
+    if constexpr(P::NSTAT == 0) {
+        hipLaunchKernelGGL((dev::k_round_nostatic<P>), dim3(1, jobs ? jobs : 1u), dim3(dev::kBlock), 0, s, stack, round,
+                           k_max, fanout, fin, spl, crit, c, block_counts, gens, job_stride);
+        return hipGetLastError();
+    }
+    return hipErrorInvalidValue;
 }
 template<class P>
 hipError_t final_nostatic(dev::BoxList fin, dev::BoxList out, unsigned long long* block_counts, unsigned grid,
@@ -248,6 +273,7 @@ KernelSet make_kernel_set(std::uint64_t fingerprint, const char* key, const doub
     k.static_level = &detail::static_level<P>;
     k.dynamic_level = &detail::dynamic_level<P>;
     k.hull_finalize = &detail::hull_finalize<P>;
+    k.round_nostatic = &detail::round_nostatic<P>;
     k.final_nostatic = &detail::final_nostatic<P>;
     k.initial_box = &detail::initial_box<P>;
     k.hull_decode = &detail::hull_decode<P>;

@@ -12,6 +12,7 @@
 #include <algorithm>
 #include <chrono>
 #include <cstdio>
+#include <cstddef>
 #include <cstring>
 #include <functional>
 #include <limits>
@@ -65,16 +66,17 @@ template<typename F> int guarded(F&& f) {
 // whole state to the host.
 struct DeviceState {
     dev::DeviceCounters counters;
-    unsigned long long stack_count, fin_count, spl_count, crit_count, scratch_count;
-    unsigned long long round_k, round_base;   // the round pops [round_base, round_base + round_k)
-    unsigned long long host_n;                // input count of host-driven calls
-    unsigned long long frontier_full;         // nonzero: a round could not pop anything
-    unsigned long long level_count[64];       // output counter of (mode, level): mode * 16 + level
     unsigned long long f32_decided;           // static-level children pruned by the FP32 prefilter
     unsigned long long f32_checked;           // static-level children the FP32 prefilter evaluated
-    unsigned long long undec_count[32];       // FP32 prefilter: undecided children of (mode, level), mode * 16 + level
+    unsigned long long stack_count, crit_count, scratch_count;
     unsigned long long part_n;                // inputs of one part of a final pass repeated in parts
+    dev::RoundWords round;
+    unsigned long long level_count[64];       // output counter of (mode, level): mode * 16 + level
+    unsigned long long undec_count[32];       // FP32 prefilter: undecided children of (mode, level), mode * 16 + level
 };
+// The counters that the end of a round clears for the next one are its last words.
+constexpr unsigned kStateWords = sizeof(DeviceState) / sizeof(unsigned long long);
+constexpr unsigned kKeptWords = kStateWords - 96;
 
 static_assert(sizeof(DeviceState) % sizeof(unsigned long long) == 0, "state is a block of 64-bit words");
 
@@ -94,44 +96,13 @@ __device__ __forceinline__ void segment_counters_reset(SegCounters s, unsigned l
 __global__ void k_set_u64(unsigned long long* p, unsigned long long v) {
     if(threadIdx.x == 0 && blockIdx.x == 0) *p = v;
 }
-// Start of a proof: the job's control block to zero and its initial runtime
-// box (computed once when the core was created, as the reference computes it
-// when it builds the prover input, refactor_constraints_impl.hpp:114) as the
-// single entry of the initial-queue input list, at depth 0.  Row blockIdx.y
-// works on job blockIdx.y.  With `start_flag` (a word per job) only the jobs
-// whose flag is set start; the others keep their state and get an empty
-// initial-queue input.
-__global__ void k_proof_start(unsigned long long* words, unsigned n_words, const double* box, int n_args,
-                              double* list_lb, double* list_ub, unsigned* list_depth, unsigned long long list_stride,
-                              unsigned long long count_word, const unsigned long long* start_flag,
-                              SegCounters segs, unsigned long long stride) {
-    const unsigned long long off = dev::job_offset(stride);
-    words = dev::job_ptr(words, off);
-    box = dev::job_ptr(box, off);
-    list_lb = dev::job_ptr(list_lb, off);
-    list_ub = dev::job_ptr(list_ub, off);
-    list_depth = dev::job_ptr(list_depth, off);
-    start_flag = dev::job_ptr(start_flag, off);
-    if(blockIdx.x != 0) return;
-    if(start_flag && *start_flag == 0ull) {
-        if(threadIdx.x == 0) words[count_word] = 0ull;
-        return;
-    }
-    for(unsigned i = threadIdx.x; i < n_words; i += blockDim.x) words[i] = 0ull;
-    for(int a = static_cast<int>(threadIdx.x); a < n_args; a += static_cast<int>(blockDim.x)) {
-        list_lb[static_cast<unsigned long long>(a) * list_stride] = box[a];
-        list_ub[static_cast<unsigned long long>(a) * list_stride] = box[n_args + a];
-    }
-    segment_counters_reset(segs, off);
-    if(threadIdx.x == 0 && list_depth) list_depth[0] = 0u;
-    __syncthreads();
-    if(threadIdx.x == 0) words[count_word] = 1ull;
-}
 // Most jobs of one batch (sqd_prove_batch).
 constexpr unsigned kMaxJobs = 64;
 // The initial-queue range of each job of a batch: [lo[j], hi[j]), and whether
 // the job starts with the next proof start (continuous batches start only the
-// rows that were admitted since the last round).
+// rows that were admitted since the last round).  The first kernel of a proof
+// reads it from pinned host memory (dev::StartArgs), so that captured graphs fit
+// every range without a launch of its own that sets it.
 struct JobRanges {
     unsigned lo[kMaxJobs];
     unsigned hi[kMaxJobs];
@@ -140,13 +111,40 @@ struct JobRanges {
 // Kernels below with a `stride` argument run one grid row per job of a batch:
 // row blockIdx.y works on job blockIdx.y's memory (job 0's pointers shifted by
 // blockIdx.y * stride bytes).
-__global__ void k_set_ranges(unsigned long long* p, unsigned long long stride, JobRanges r) {
-    p = dev::job_ptr(p, dev::job_offset(stride));
-    if(threadIdx.x == 0 && blockIdx.x == 0) {
-        p[0] = r.lo[blockIdx.y];
-        p[1] = r.hi[blockIdx.y];
-        p[2] = r.start[blockIdx.y];
+// Start of a proof where the initial queue's first level cannot do it
+// (dev::StartArgs; without pinned memory the ranges come as an argument): the
+// job's control block to zero, its range to `range` and its initial runtime box
+// (computed once when the core was created, as the reference computes it when it
+// builds the prover input, refactor_constraints_impl.hpp:114) as the single entry
+// of the initial-queue input list, at depth 0.  Row blockIdx.y works on job
+// blockIdx.y; jobs that do not start get an empty initial-queue input.
+__global__ void k_proof_start(dev::StartArgs s, JobRanges given, unsigned from_host, int n_args, dev::BoxList list,
+                              unsigned long long* range, unsigned long long stride) {
+    const unsigned long long off = dev::job_offset(stride);
+    unsigned long long* words = dev::job_ptr(s.words, off);
+    const double* box = dev::job_ptr(s.box, off);
+    list = dev::job_list(list, off);
+    range = dev::job_ptr(range, off);
+    if(blockIdx.x != 0) return;
+    const unsigned j = blockIdx.y;
+    const unsigned lo = from_host ? s.host_ranges[j] : given.lo[j], hi = from_host ? s.host_ranges[64 + j] : given.hi[j];
+    if(s.flagged && !(from_host ? s.host_ranges[128 + j] : given.start[j])) {
+        if(threadIdx.x == 0) *list.count = 0ull;
+        return;
     }
+    for(unsigned i = threadIdx.x; i < s.n_words; i += blockDim.x) words[i] = 0ull;
+    for(int a = static_cast<int>(threadIdx.x); a < n_args; a += static_cast<int>(blockDim.x)) {
+        list.lb[static_cast<unsigned long long>(a) * list.stride] = box[a];
+        list.ub[static_cast<unsigned long long>(a) * list.stride] = box[n_args + a];
+    }
+    segment_counters_reset(SegCounters{s.seg_counters, s.seg_lists}, off);
+    if(threadIdx.x == 0) {
+        if(list.depth) list.depth[0] = 0u;
+        range[0] = lo;
+        range[1] = hi;
+    }
+    __syncthreads();
+    if(threadIdx.x == 0) *list.count = 1ull;
 }
 // Start of a proof (or of a host-driven call): the whole control block (state
 // and per-block count slots) to zero.
@@ -156,76 +154,60 @@ __global__ void k_state_reset(unsigned long long* words, unsigned long long n_wo
     if(blockIdx.x == 0) segment_counters_reset(segs, dev::job_offset(stride));
     for(unsigned long long i = threadIdx.x; blockIdx.x == 0 && i < n_words; i += blockDim.x) words[i] = 0ull;
 }
-// The control blocks of a batch's jobs side by side in `out` (one copy to the host).
-__global__ void k_gather_states(const unsigned long long* st, unsigned long long stride, unsigned long long* out,
-                                unsigned words) {
-    st = dev::job_ptr(st, dev::job_offset(stride));
-    for(unsigned i = threadIdx.x; blockIdx.x == 0 && i < words; i += blockDim.x)
-        out[static_cast<unsigned long long>(blockIdx.y) * words + i] = st[i];
-}
-// Start of a round: pop K = min(k_max, S, room / (fanout - 1)) cuboids from
-// the top of the stack (their slots are reused by the children the round
-// pushes), and clear the round's list counters.
-__global__ void k_round_begin(DeviceState* st, unsigned long long k_max, unsigned long long stack_cap,
-                              unsigned long long fanout, SegCounters segs, unsigned long long stride) {
-    st = dev::job_ptr(st, dev::job_offset(stride));
-    const unsigned t = threadIdx.x;
-    if(blockIdx.x != 0) return;
-    segment_counters_reset(segs, dev::job_offset(stride));
-    if(t == 0) {
-        const unsigned long long S = st->stack_count;
-        unsigned long long K = S < k_max ? S : k_max;
-        if(fanout > 1) {
-            const unsigned long long room = stack_cap > S ? stack_cap - S : 0;
-            const unsigned long long lim = room / (fanout - 1);
-            K = K < lim ? K : lim;
-        }
-        if(K == 0 && S > 0) st->frontier_full = 1;
-        st->round_k = K;
-        st->round_base = S - K;
-        st->stack_count = S - K;
-        st->fin_count = 0;
-        st->spl_count = 0;
-    }
-    if(t < 64) st->level_count[t] = 0;
-    if(t < 32) st->undec_count[t] = 0;
-}
-// Adds the per-block count slots into the state's counters and clears them
-// (run before the state is read).  Each block folds kFoldThreads slots of its
-// job (one per thread), reduces them across its waves and adds the sums to the
-// counters with atomics, so that the slots are read by many compute units at
-// once instead of one.
-constexpr unsigned kFoldThreads = 256;
-__global__ __launch_bounds__(kFoldThreads) void k_fold_counts(DeviceState* st, unsigned long long* slots,
-                                                              unsigned long long n_slots, unsigned long long stride) {
-    st = dev::job_ptr(st, dev::job_offset(stride));
-    slots = dev::job_ptr(slots, dev::job_offset(stride));
+// End of a round (or of a host-driven call), one block per job: adds the
+// per-block count slots into the state's counters and clears them, brings the
+// whole state to the host (`host`: pinned memory, one state per job; nullptr: the
+// caller copies it) and clears the level counters for the next round.  Two
+// kernels (fold, gather) and a copy did this before, at 4 to 5 us each.
+constexpr unsigned kEndThreads = 1024;
+__global__ __launch_bounds__(kEndThreads) void k_round_end(DeviceState* st, unsigned long long* slots,
+                                                           unsigned long long n_slots, SegCounters segs,
+                                                           DeviceState* host, unsigned long long* done,
+                                                           unsigned long long ticket, unsigned long long stride) {
+    const unsigned long long off = dev::job_offset(stride);
+    st = dev::job_ptr(st, off);
+    slots = dev::job_ptr(slots, off);
     constexpr int W = 5;   // used words of a slot
-    __shared__ unsigned long long part[W][kFoldThreads / 64];
+    __shared__ unsigned long long part[W][kEndThreads / 64];
     unsigned long long acc[W] = {0, 0, 0, 0, 0};
-    for(unsigned long long i = static_cast<unsigned long long>(blockIdx.x) * blockDim.x + threadIdx.x; i < n_slots;
-        i += static_cast<unsigned long long>(gridDim.x) * blockDim.x) {
+    for(unsigned long long i = threadIdx.x; i < n_slots; i += kEndThreads) {
         unsigned long long* s = slots + static_cast<unsigned long long>(dev::kSlotWords) * i;
         unsigned long long v[W];
 #pragma unroll
         for(int j = 0; j < W; ++j) v[j] = s[j];
 #pragma unroll
-        for(int j = 0; j < W; ++j) { acc[j] += v[j]; s[j] = 0ull; }
+        for(int j = 0; j < W; ++j) {
+            acc[j] += v[j];
+            if(v[j]) s[j] = 0ull;
+        }
     }
+    unsigned long long* const words = reinterpret_cast<unsigned long long*>(st);
+    unsigned long long* const out = host ? reinterpret_cast<unsigned long long*>(host + blockIdx.y) : nullptr;
+    const unsigned w = threadIdx.x;   // the thread's word of the state
+    static_assert(kStateWords <= kEndThreads && offsetof(DeviceState, counters) == 0 &&
+                  offsetof(DeviceState, f32_decided) == 4 * sizeof(unsigned long long), "counters first");
+    unsigned long long v = w < kStateWords ? words[w] : 0ull;
 #pragma unroll
-    for(int j = 0; j < W; ++j) acc[j] = dev::wave_sum(acc[j]);
-    if(__lane_id() == 0)
-        for(int j = 0; j < W; ++j) part[j][threadIdx.x / 64] = acc[j];
+    for(int j = 0; j < W; ++j) {
+        acc[j] = dev::wave_sum(acc[j]);
+        if(__lane_id() == 0) part[j][threadIdx.x / 64] = acc[j];
+    }
+    segment_counters_reset(segs, off);
     __syncthreads();
-    if(threadIdx.x == 0) {
-        unsigned long long sum[W] = {0, 0, 0, 0, 0};
-        for(unsigned w = 0; w < blockDim.x / 64; ++w)
-            for(int j = 0; j < W; ++j) sum[j] += part[j][w];
-        if(sum[0]) atomicAdd(&st->counters.cuboids, sum[0]);
-        if(sum[1]) atomicAdd(&st->counters.leaves, sum[1]);
-        if(sum[2]) atomicAdd(&st->counters.criticals, sum[2]);
-        if(sum[3]) atomicAdd(&st->f32_decided, sum[3]);
-        if(sum[4]) atomicAdd(&st->f32_checked, sum[4]);
+    // cuboids, leaves, criticals, (overflow), decided and checked by the prefilter
+    if(w < 6 && w != 3) {
+        for(unsigned k = 0; k < kEndThreads / 64; ++k) v += part[w < 3 ? w : w - 1][k];
+        words[w] = v;
+    }
+    if(w < kStateWords && out) __hip_atomic_store(out + w, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if(w >= kKeptWords && w < kStateWords) words[w] = 0ull;
+    if(done) {
+        // tells a host that polls that its copy of the job's state is complete: the
+        // barrier waits for the stores above, which go past the caches to the
+        // (coherent) host memory; a system fence would write back the whole L2,
+        // 8 us where a level left its list there
+        __syncthreads();
+        if(w == 0) __hip_atomic_store(done + blockIdx.y, ticket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
 // Level counters to zero (between chunks of a host-driven call).
@@ -366,7 +348,9 @@ struct sqd_core {
     unsigned states = 1;                    // jobs whose state the last copy to h_state holds
     unsigned long long job_stride = 0;      // bytes of one job's part of d_jobs
     char* d_jobs = nullptr;                 // the jobs' memory, jobs parts
-    unsigned long long* d_gather = nullptr; // jobs control blocks side by side (k_gather_states)
+    sqd::JobRanges* h_ranges = nullptr;     // pinned: the jobs' ranges, read by the first kernel of a proof
+    unsigned long long* h_done = nullptr;   // pinned: the jobs' last tickets (wait_done)
+    unsigned long long tickets = 0;         // tickets given out
     unsigned long long* d_slots = nullptr;
     unsigned long long n_slots = 0;        // >= the largest grid of a counting kernel
     unsigned long long* d_discard = nullptr;   // count slots that are never folded (final passes repeated in parts)
@@ -377,6 +361,7 @@ struct sqd_core {
     sqd::SegCounters segs{nullptr, 0};   // (job) counters of the segmented level lists (none: dense lists)
     sqd::SegIndex seg_index{};           // their (mode, level)s
     unsigned char* d_has = nullptr;
+    sqd::JobRanges ranges{};                // the ranges of the next initial queues
     sqd::DevList stack, lvl[2], fin, spl, crit, scratch;
     std::uint64_t device_bytes = 0;  // device memory allocated by sqd_core_create
     sqd_critical_fn crit_fn = nullptr;       // critical sink (sqd_core_set_critical_sink)
@@ -513,39 +498,30 @@ void enqueue_level_totals(sqd_core* c) {
         return hipGetLastError();
     });
 }
-// Enqueues the fold of the count slots into the counters and the copy of the
-// device state (of every job of the launches' rows) to its pinned host copy.
-void enqueue_state_copy(sqd_core* c) {
+// Enqueues the end of a round: the count slots into the counters and the device
+// state (of every job of the launches' rows) to its host copy.
+// With a `ticket` the kernel stores it to the job's word of h_done when its copy is
+// complete (wait_done).
+void enqueue_state_copy(sqd_core* c, unsigned long long ticket = 0) {
     if(c->profiling) enqueue_level_totals(c);
-    launch(c, KIND_SET_COUNT, "k_fold_counts", [&] {
-        const unsigned blocks = static_cast<unsigned>((c->n_slots + kFoldThreads - 1) / kFoldThreads);
-        hipLaunchKernelGGL(k_fold_counts, dim3(blocks, c->ny), dim3(kFoldThreads), 0, c->stream, c->d_state, c->d_slots, c->n_slots,
+    launch(c, KIND_SET_COUNT, "k_round_end", [&] {
+        hipLaunchKernelGGL(k_round_end, dim3(1, c->ny), dim3(kEndThreads), 0, c->stream, c->d_state, c->d_slots, c->n_slots,
+                           c->segs, c->h_ranges ? c->h_state : nullptr, ticket ? c->h_done : nullptr, ticket,
                            c->job_stride);
         return hipGetLastError();
     });
-    if(c->ny == 1) {
+    if(!c->h_ranges)   // no pinned memory (sqd_prove_range_noalloc)
         hip_check(hipMemcpyAsync(c->h_state, c->d_state, sizeof(DeviceState), hipMemcpyDeviceToHost, c->stream),
                   "copy state");
-        return;
-    }
-    constexpr unsigned words = sizeof(DeviceState) / sizeof(unsigned long long);
-    launch(c, KIND_SET_COUNT, "k_gather_states", [&] {
-        hipLaunchKernelGGL(k_gather_states, dim3(1, c->ny), dim3(256), 0, c->stream,
-                           reinterpret_cast<const unsigned long long*>(c->d_state), c->job_stride, c->d_gather, words);
-        return hipGetLastError();
-    });
-    hip_check(hipMemcpyAsync(c->h_state, c->d_gather, sizeof(DeviceState) * c->ny, hipMemcpyDeviceToHost, c->stream),
-              "copy states");
 }
 // Waits for the state copy enqueued last and checks the overflow flags (of
 // every job: one failing job fails the whole call).
-const DeviceState& finish_state(sqd_core* c) {
-    sync(c);
+const DeviceState& check_state(sqd_core* c) {
     c->states = c->ny;
     for(unsigned j = 0; j < c->ny; ++j) {
         if(c->h_state[j].counters.overflow)
             throw Failure(SQD_ERR_CAPACITY, "a device level buffer overflowed; raise sqd_settings.level_bytes");
-        if(c->h_state[j].frontier_full)
+        if(c->h_state[j].round.frontier_full)
             throw Failure(SQD_ERR_CAPACITY, "frontier capacity exhausted; raise sqd_settings.frontier_capacity");
         if(c->h_state[j].crit_count > c->crit.cap && !(c->crit_fn && c->ny == 1))
             throw Failure(SQD_ERR_CAPACITY, "more critical cuboids (" + std::to_string(c->h_state[j].crit_count) +
@@ -555,6 +531,30 @@ const DeviceState& finish_state(sqd_core* c) {
     }
     return *c->h_state;
 }
+const DeviceState& finish_state(sqd_core* c) {
+    sync(c);
+    return check_state(c);
+}
+// The same for a state copy with a ticket: polls the jobs' words in pinned memory
+// instead of waiting for the stream (One 65.5 against 71 us a proof, Two 111 either
+// way), and looks at the stream every few milliseconds, which reports a kernel
+// that failed (a look costs 8 to 15 us).
+const DeviceState& wait_done(sqd_core* c, unsigned long long ticket) {
+    constexpr std::chrono::milliseconds kLook{5};
+    auto look = std::chrono::steady_clock::now() + kLook;
+    for(unsigned j = 0; j < c->ny; ++j)
+        for(unsigned spins = 1; __atomic_load_n(c->h_done + j, __ATOMIC_ACQUIRE) != ticket; ++spins) {
+            if(spins % 256 == 0 && std::chrono::steady_clock::now() > look) {
+                const hipError_t e = hipStreamQuery(c->stream);
+                if(e == hipSuccess) return finish_state(c);   // all done: the copies are complete
+                if(e != hipErrorNotReady) hip_check(e, "hipStreamQuery");
+                look = std::chrono::steady_clock::now() + kLook;
+            }
+            __builtin_ia32_pause();
+        }
+    return check_state(c);
+}
+
 // With profiling on: adds the child cuboids of the round whose state was copied
 // last to the statistics of the level kernels that timed them.  A static level's
 // children are its inputs times its subdivisions; the inputs of level 0 are the
@@ -570,13 +570,13 @@ void count_children(sqd_core* c) {
     for(unsigned j = 0; j < c->ny; ++j) {
         const DeviceState& h = c->h_state[j];
         for(int mode : {dev::NONFINAL, dev::FINAL}) {
-            unsigned long long in = mode == dev::NONFINAL ? h.round_k : h.fin_count;
+            unsigned long long in = mode == dev::NONFINAL ? h.round.round_k : h.round.fin_count;
             for(int L = 0; L < S; ++L) {
                 add(mode * 16 + L, in * c->st_subs[static_cast<std::size_t>(L)]);
                 in = h.level_count[mode * 16 + L];
             }
         }
-        unsigned long long in = h.spl_count;
+        unsigned long long in = h.round.spl_count;
         for(int J = 0; J < D; ++J) {
             add(dev::SPLIT * 16 + J, in * c->dyn_subs[static_cast<std::size_t>(J)]);
             in = h.level_count[dev::SPLIT * 16 + J];
@@ -623,6 +623,9 @@ dev::LevelArgs level_args(sqd_core* c, const dev::BoxList& in, const unsigned lo
     a.children_per_lane = static_cast<int>(std::min<uint32_t>(c->settings.prefilter_group, 64u));
     a.job_stride = c->job_stride;
     a.jobs = c->ny;
+    a.pop = nullptr;
+    a.pop_max = c->k_max;
+    a.pop_fanout = c->split_fanout;
     return a;
 }
 
@@ -643,6 +646,7 @@ void run_static_level(sqd_core* c, int mode, int L, const dev::BoxList& in, cons
     dev::BoxList src = in;
     if(L == 0) { src.origin = nullptr; src.leaf = nullptr; }  // the input index is the origin
     dev::LevelArgs a = level_args(c, src, base, count, out);
+    if(count == &c->d_state->round.round_k) a.pop = &c->d_state->round;   // a round's first level takes its cuboids
     a.undec_count = &c->d_state->undec_count[mode * 16 + L];
     // the group test: sized by the settings on the levels that ask for one (here or
     // in the prefilter), by the kernel on the last level of a plain proof; off
@@ -689,7 +693,7 @@ void run_static(sqd_core* c, int mode, const dev::BoxList& in, const unsigned lo
 // Dynamic levels (SPLIT or INIT) from the inputs [0, *count) of `in` (at most
 // `max_items`) to `out`, appending to its counter.
 void run_dynamic(sqd_core* c, int mode, const dev::BoxList& in, const unsigned long long* count,
-                 unsigned long long max_items, const dev::BoxList& out) {
+                 unsigned long long max_items, const dev::BoxList& out, const dev::StartArgs& start = {}) {
     const int D = c->ks->NDYN;
     dev::BoxList prev = in;
     const unsigned long long* prev_count = count;
@@ -706,7 +710,7 @@ void run_dynamic(sqd_core* c, int mode, const dev::BoxList& in, const unsigned l
         const unsigned long long children =
             items * (mode == dev::INIT ? c->dyn_initial[static_cast<std::size_t>(J)] : c->dyn_subs[static_cast<std::size_t>(J)]);
         launch(c, mode * 16 + J, "dynamic level launch",
-               [&] { return c->ks->dynamic_level(mode, J, a, children, c->cus, c->grid_override, c->stream); });
+               [&] { return c->ks->dynamic_level(mode, J, a, J == 0 ? start : dev::StartArgs{}, children, c->cus, c->grid_override, c->stream); });
         prev = o;
         prev_count = o.count;
         items = std::min<unsigned long long>(children, c->lvl[J % 2].cap);
@@ -800,10 +804,8 @@ void launch_initial_box(sqd_core* c, bool to_scratch, bool reset) {
 // The ranges of the first dynamic variable's initial subdivisions that the next
 // initial queues (one per job of the launches' rows) start from.
 void set_ranges(sqd_core* c, const JobRanges& r) {
-    launch(c, KIND_SET_COUNT, "k_set_ranges", [&] {
-        hipLaunchKernelGGL(k_set_ranges, dim3(1, c->ny), dim3(64), 0, c->stream, c->d_range, c->job_stride, r);
-        return hipGetLastError();
-    });
+    c->ranges = r;
+    if(c->h_ranges) *c->h_ranges = r;   // read by the proof's first kernel; no earlier one is in flight
 }
 void set_range(sqd_core* c, unsigned long long first, unsigned long long last) {
     JobRanges r{};
@@ -814,21 +816,26 @@ void set_range(sqd_core* c, unsigned long long first, unsigned long long last) {
 unsigned long long full_range(const sqd_core* c) { return c->dyn_initial.empty() ? 1ull : c->dyn_initial[0]; }
 
 // Enqueues a cleared device state and the initial queue on the (empty) stack;
-// nothing is waited for.  The initial box is the one computed when the core
-// was created (d_box_init).
+// nothing is waited for.  The initial box is the one computed when the core was
+// created (d_box_init).  The initial queue's first level does the start itself
+// where its children fit one block and the core has pinned memory.
 void enqueue_initial_queue(sqd_core* c, bool only_flagged = false) {
-    launch(c, KIND_INITIAL_BOX, "proof start", [&] {
-        const unsigned words = static_cast<unsigned>(sizeof(DeviceState) / sizeof(unsigned long long));
-        const unsigned long long count_word =
-            static_cast<unsigned long long>(reinterpret_cast<char*>(c->scratch.count) - reinterpret_cast<char*>(c->d_state)) /
-            sizeof(unsigned long long);
-        hipLaunchKernelGGL(k_proof_start, dim3(1, c->ny), dim3(64), 0, c->stream,
-                           reinterpret_cast<unsigned long long*>(c->d_state), words, c->d_box_init, c->N, c->scratch.lb,
-                           c->scratch.ub, c->scratch.depth, c->scratch.cap, count_word,
-                           only_flagged ? c->d_range + 2 : nullptr, c->segs, c->job_stride);
-        return hipGetLastError();
-    });
-    run_dynamic(c, dev::INIT, c->scratch.view(), c->scratch.count, 1, c->stack.view());
+    const bool fused = c->h_ranges && c->ks->NDYN > 0 && c->dyn_initial[0] <= dev::kBlock;
+    dev::StartArgs s{};
+    s.words = reinterpret_cast<unsigned long long*>(c->d_state);
+    s.n_words = kStateWords;
+    s.box = c->d_box_init;
+    s.host_ranges = c->h_ranges ? c->h_ranges->lo : nullptr;
+    s.flagged = only_flagged ? 1u : 0u;
+    s.seg_counters = c->segs.p;
+    s.seg_lists = c->segs.n_lists;
+    if(!fused)
+        launch(c, KIND_INITIAL_BOX, "proof start", [&] {
+            hipLaunchKernelGGL(k_proof_start, dim3(1, c->ny), dim3(64), 0, c->stream, s, c->ranges, c->h_ranges ? 1u : 0u,
+                               c->N, c->scratch.view(), c->d_range, c->job_stride);
+            return hipGetLastError();
+        });
+    run_dynamic(c, dev::INIT, c->scratch.view(), c->scratch.count, 1, c->stack.view(), fused ? s : dev::StartArgs{});
 }
 
 // Calls the core's progress callback with the last state brought to the host.
@@ -882,30 +889,38 @@ template<typename F> hipGraphExec_t capture_graph(sqd_core* c, F&& enqueue) {
     return e;
 }
 
-// Enqueues one round over the top of the stack: pop (on the device), non-final
-// static levels with hull join, hull sorting into final and split lists, final
-// pass, dynamic split pushing the children.  Nothing is waited for.
-void enqueue_round(sqd_core* c) {
+// The parts of a round over the top of the stack; nothing is waited for.
+// First part: the round's cuboids are taken (on the device), the non-final static
+// levels join their hulls, and the hulls are sorted into the final and split lists.
+void enqueue_nonfinal(sqd_core* c) {
     DeviceState* st = c->d_state;
-    launch(c, KIND_SET_COUNT, "k_round_begin", [&] {
-        hipLaunchKernelGGL(k_round_begin, dim3(1, c->ny), dim3(64), 0, c->stream, st, c->k_max, c->stack.cap,
-                           c->split_fanout, c->segs, c->job_stride);
-        return hipGetLastError();
-    });
     const unsigned long long K = c->k_max;   // bound on the round's size
     dev::BoxList items = c->stack.view();
-    if(c->ks->NSTAT > 0) run_static(c, dev::NONFINAL, items, &st->round_base, &st->round_k, K, c->crit.view());
+    if(c->ks->NSTAT == 0) {   // (finishes the last generation's cuboids too)
+        launch(c, KIND_HULL_FINALIZE, "round without static levels", [&] {
+            return c->ks->round_nostatic(items, &st->round, c->k_max, c->split_fanout, c->fin.view(), c->spl.view(),
+                                         c->crit.view(), &st->counters, c->d_slots, c->settings.generation_count, c->ny,
+                                         c->job_stride, c->stream);
+        });
+        return;
+    }
+    run_static(c, dev::NONFINAL, items, &st->round.round_base, &st->round.round_k, K, c->crit.view());
     launch(c, KIND_HULL_FINALIZE, "hull finalize", [&] {
-        return c->ks->hull_finalize(items, &st->round_base, &st->round_k, K, c->d_hull, c->fin.view(), c->spl.view(),
-                                    &st->counters, c->d_slots, c->settings.generation_count, c->ny, c->job_stride,
+        return c->ks->hull_finalize(items, &st->round.round_base, &st->round.round_k, K, c->d_hull, c->fin.view(),
+                                    c->spl.view(), &st->counters, c->settings.generation_count, c->ny, c->job_stride,
                                     c->stream);
     });
-    if(c->ks->NSTAT > 0) run_static(c, dev::FINAL, c->fin.view(), nullptr, c->fin.count, K, c->crit.view());
-    else launch(c, KIND_FINAL_NOSTATIC, "final", [&] {
-        return c->ks->final_nostatic(c->fin.view(), c->crit.view(), c->d_slots,
-                                     static_cast<unsigned>((K + 255) / 256), c->ny, c->job_stride, c->stream);
-    });
-    run_dynamic(c, dev::SPLIT, c->spl.view(), c->spl.count, K, c->stack.view());
+}
+// Second part: the final pass over the final list.
+void enqueue_final(sqd_core* c) {
+    if(c->ks->NSTAT > 0) run_static(c, dev::FINAL, c->fin.view(), nullptr, c->fin.count, c->k_max, c->crit.view());
+}
+// Third part: the dynamic split of the split list pushes the children.
+void enqueue_split(sqd_core* c) { run_dynamic(c, dev::SPLIT, c->spl.view(), c->spl.count, c->k_max, c->stack.view()); }
+void enqueue_round(sqd_core* c) {
+    enqueue_nonfinal(c);
+    enqueue_final(c);
+    enqueue_split(c);
 }
 
 // Hands the criticals [0, k) of the critical list (k <= its capacity) to the sink.
@@ -1008,7 +1023,61 @@ void track_peaks(sqd_core* c) {
 void drain_round(sqd_core* c) {
     if(!c->crit_fn || c->ny != 1) return;
     const DeviceState& h = c->h_state[0];
-    if(h.crit_count) drain_criticals(c, h.crit_count, h.fin_count);
+    if(h.crit_count) drain_criticals(c, h.crit_count, h.round.fin_count);
+}
+
+// The rounds of a proof, each in steps that end where the host looks at the
+// state: after the hulls are sorted.  A step is the final pass and the split of
+// the round before, where some job's lists hold anything for them, and the first
+// part of the next round; a proof whose cuboids all die in their first round
+// (One to Four, More2) never launches a final or split level.  An empty level
+// costs its 4.5 us all the same: 3 of them per round for One, 8 for Six.
+// Without static levels every cuboid is its own hull, so that there is always
+// something to split: whole rounds.
+//
+// The steps are launched directly: a captured graph of the same six to nine
+// kernels starts later (its first kernel waits for the whole graph to be put in
+// the queue): One 70 against 75 us, Three 175 against 180, Four 753 against 762.
+void prove_steps(sqd_core* c) {
+    enum : unsigned { FIN = 1, SPL = 2, NEXT = 4 };
+    auto run = [&](auto&& enqueue) {
+        enqueue();
+        if(!c->h_done) {
+            enqueue_state_copy(c);
+            finish_state(c);
+            return;
+        }
+        const unsigned long long ticket = ++c->tickets;
+        enqueue_state_copy(c, ticket);
+        wait_done(c, ticket);
+    };
+    if(c->ks->NSTAT == 0) {
+        run([&] { enqueue_initial_queue(c); enqueue_round(c); });
+        track_peaks(c);
+        while(frontier_left(c)) {
+            run([&] { enqueue_round(c); });
+            track_peaks(c);
+        }
+        return;
+    }
+    run([&] { enqueue_initial_queue(c); enqueue_nonfinal(c); });
+    for(;;) {
+        unsigned parts = 0;
+        for(unsigned j = 0; j < c->ny; ++j) {
+            const DeviceState& h = c->h_state[j];
+            if(h.round.fin_count) parts |= FIN;
+            if(h.round.spl_count) parts |= SPL | NEXT;
+            if(h.stack_count) parts |= NEXT;
+        }
+        if(!parts) break;
+        run([&] {
+            if(parts & FIN) enqueue_final(c);
+            if(parts & SPL) enqueue_split(c);
+            if(parts & NEXT) enqueue_nonfinal(c);
+        });
+        if(!(parts & NEXT)) break;   // (the lists keep the counts of what was done)
+    }
+    for(unsigned j = 0; j < c->ny; ++j) c->row_peak[j] = c->h_state[j].round.frontier_peak;
 }
 
 // Proves the initial ranges [first[j], last[j]) of n jobs, leaving each job's
@@ -1041,6 +1110,13 @@ void prove_jobs(sqd_core* c, unsigned n, const uint32_t* first, const uint32_t* 
     c->crit_delivered = 0;
     c->row_peak.assign(c->ny, 0ull);
     const bool graphs = c->settings.graphs && !c->profiling && c->proofs > 0;
+    if(!c->profiling && !c->crit_fn && !(progress_reports && c->progress_fn)) {
+        prove_steps(c);
+        ++c->proofs;
+        end_call(c);
+        if(seconds) *seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
+        return;
+    }
     if(graphs && !c->g_first) {
         c->g_first = capture_graph(c, [&] { enqueue_initial_queue(c); enqueue_round(c); enqueue_state_copy(c); });
         c->g_round = capture_graph(c, [&] { enqueue_round(c); enqueue_state_copy(c); });
@@ -1236,8 +1312,8 @@ void bind_state(sqd_core* c, unsigned long long* state_words) {
     c->level_slots = c->d_slots;
     DeviceState* st = c->d_state;
     c->stack.count = &st->stack_count;
-    c->fin.count = &st->fin_count;
-    c->spl.count = &st->spl_count;
+    c->fin.count = &st->round.fin_count;
+    c->spl.count = &st->round.spl_count;
     c->crit.count = &st->crit_count;
     c->scratch.count = &st->scratch_count;
 }
@@ -1382,11 +1458,13 @@ int sqd_core_create(int device, const sqd_program* program, const sqd_settings* 
         c->d_jobs = dalloc<char>(static_cast<std::size_t>(c->job_stride) * c->jobs);
         lay.place(c->d_jobs);
         bind_state(c.get(), state_words);
-        if(c->jobs > 1) c->d_gather = dalloc<unsigned long long>(sizeof(DeviceState) / sizeof(unsigned long long) * c->jobs);
         void* hs = nullptr;
-        hip_check(hipHostMalloc(&hs, sizeof(DeviceState) * c->jobs, hipHostMallocDefault), "hipHostMalloc");
+        const std::size_t host_bytes = sizeof(DeviceState) * c->jobs + sizeof(unsigned long long) * c->jobs + sizeof(JobRanges);
+        hip_check(hipHostMalloc(&hs, host_bytes, hipHostMallocMapped | hipHostMallocCoherent), "hipHostMalloc");
         c->h_state = static_cast<DeviceState*>(hs);
-        std::memset(c->h_state, 0, sizeof(DeviceState) * c->jobs);
+        std::memset(hs, 0, host_bytes);
+        c->h_done = reinterpret_cast<unsigned long long*>(c->h_state + c->jobs);
+        c->h_ranges = reinterpret_cast<JobRanges*>(c->h_done + c->jobs);
         upload_job_constants(c.get());
         compute_initial_boxes(c.get());
         hip_check(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
@@ -1400,8 +1478,7 @@ void sqd_core_destroy(sqd_core* c) {
     std::lock_guard<std::mutex> lock(g_capture_mutex);
     (void)hipSetDevice(c->device);
     if(c->stream) (void)hipStreamSynchronize(c->stream);
-    for(void* p : {static_cast<void*>(c->d_jobs), static_cast<void*>(c->d_gather)})
-        if(p) (void)hipFree(p);
+    if(c->d_jobs) (void)hipFree(c->d_jobs);
     if(c->h_state) (void)hipHostFree(c->h_state);
     if(c->g_first) (void)hipGraphExecDestroy(c->g_first);
     if(c->g_round) (void)hipGraphExecDestroy(c->g_round);
