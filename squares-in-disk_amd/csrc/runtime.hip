@@ -210,6 +210,26 @@ __global__ __launch_bounds__(kEndThreads) void k_round_end(DeviceState* st, unsi
         if(w == 0) __hip_atomic_store(done + blockIdx.y, ticket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
+// Boxes that a caller hands over, from pinned host memory (N * n lower, then N * n
+// upper bounds) into a device list, with its count and depth, by reading them
+// over the bus: 2 N copies of a few KB took 10 to 15 us each.  The first block
+// clears the level counters (and, with `whole`, the whole state) first.
+__global__ __launch_bounds__(256) void k_load_boxes(dev::BoxList list, const double* src, unsigned long long n, unsigned n_args,
+                                                    unsigned depth, DeviceState* st, unsigned whole, SegCounters segs) {
+    const unsigned long long half = n * n_args;
+    for(unsigned long long k = static_cast<unsigned long long>(blockIdx.x) * blockDim.x + threadIdx.x; k < 2 * half;
+        k += static_cast<unsigned long long>(gridDim.x) * blockDim.x) {
+        const unsigned long long at = k < half ? k : k - half;
+        (k < half ? list.lb : list.ub)[at / n * list.stride + at % n] = src[k];
+        if(list.depth && k < n) list.depth[k] = depth;
+    }
+    if(blockIdx.x != 0) return;
+    unsigned long long* const words = reinterpret_cast<unsigned long long*>(st);
+    for(unsigned i = (whole ? 0u : kKeptWords) + threadIdx.x; i < kStateWords; i += blockDim.x) words[i] = 0ull;
+    segment_counters_reset(segs, 0ull);
+    __syncthreads();
+    if(threadIdx.x == 0) *list.count = n;
+}
 // Level counters to zero (between chunks of a host-driven call).
 __global__ void k_levels_reset(DeviceState* st, SegCounters segs) {
     if(blockIdx.x == 0) segment_counters_reset(segs, 0ull);
@@ -351,6 +371,8 @@ struct sqd_core {
     sqd::JobRanges* h_ranges = nullptr;     // pinned: the jobs' ranges, read by the first kernel of a proof
     unsigned long long* h_done = nullptr;   // pinned: the jobs' last tickets (wait_done)
     unsigned long long tickets = 0;         // tickets given out
+    char* h_stage = nullptr;                // pinned: boxes on their way to and from host-driven calls
+    std::size_t stage_bytes = 0;
     unsigned long long* d_slots = nullptr;
     unsigned long long n_slots = 0;        // >= the largest grid of a counting kernel
     unsigned long long* d_discard = nullptr;   // count slots that are never folded (final passes repeated in parts)
@@ -360,7 +382,6 @@ struct sqd_core {
     unsigned clean = 0;               // jobs (from 0) whose hull records and count slots are known reset
     sqd::SegCounters segs{nullptr, 0};   // (job) counters of the segmented level lists (none: dense lists)
     sqd::SegIndex seg_index{};           // their (mode, level)s
-    unsigned char* d_has = nullptr;
     sqd::JobRanges ranges{};                // the ranges of the next initial queues
     sqd::DevList stack, lvl[2], fin, spl, crit, scratch;
     std::uint64_t device_bytes = 0;  // device memory allocated by sqd_core_create
@@ -592,8 +613,13 @@ bool frontier_left(const sqd_core* c) {
 }
 // Folds the count slots and brings the device state to the host (one copy, one sync).
 const DeviceState& read_state(sqd_core* c) {
-    enqueue_state_copy(c);
-    return finish_state(c);
+    if(!c->h_done || c->profiling) {
+        enqueue_state_copy(c);
+        return finish_state(c);
+    }
+    const unsigned long long ticket = ++c->tickets;
+    enqueue_state_copy(c, ticket);
+    return wait_done(c, ticket);
 }
 sqd_counts counts_of(const DeviceState& h) {
     sqd_counts r;
@@ -717,21 +743,41 @@ void run_dynamic(sqd_core* c, int mode, const dev::BoxList& in, const unsigned l
     }
 }
 
-void upload_soa(sqd_core* c, DevList& l, const double* lb, const double* ub, unsigned long long n, unsigned depth) {
+// At least `bytes` of the core's pinned staging memory (grown as calls need it).
+char* stage(sqd_core* c, std::size_t bytes) {
+    if(bytes > c->stage_bytes) {
+        std::lock_guard<std::mutex> lock(g_capture_mutex);
+        if(c->h_stage) (void)hipHostFree(c->h_stage);
+        c->h_stage = nullptr;
+        c->stage_bytes = 0;
+        std::size_t want = 64 << 10;
+        while(want < bytes) want *= 2;
+        void* p = nullptr;
+        hip_check(hipHostMalloc(&p, want, hipHostMallocMapped | hipHostMallocCoherent), "hipHostMalloc");
+        c->h_stage = static_cast<char*>(p);
+        c->stage_bytes = want;
+    }
+    return c->h_stage;
+}
+// n boxes (SoA with stride `stride`) into list l, through the staging memory.
+// `whole`: the control block is cleared first (else only the level counters).
+// `extra` bytes of the staging memory behind the boxes are kept for the caller.
+// Nothing is waited for; no launch that reads the staging memory is in flight.
+void load_boxes(sqd_core* c, const DevList& l, const double* lb, const double* ub, std::size_t n, std::size_t stride,
+                unsigned depth, bool whole, std::size_t extra = 0) {
     if(n > l.cap) throw Failure(SQD_ERR_CAPACITY, "input larger than the device list");
-    for(int a = 0; a < c->N; ++a) {
-        hip_check(hipMemcpyAsync(l.lb + static_cast<std::size_t>(a) * l.cap, lb + static_cast<std::size_t>(a) * n,
-                                 n * sizeof(double), hipMemcpyHostToDevice, c->stream), "upload lb");
-        hip_check(hipMemcpyAsync(l.ub + static_cast<std::size_t>(a) * l.cap, ub + static_cast<std::size_t>(a) * n,
-                                 n * sizeof(double), hipMemcpyHostToDevice, c->stream), "upload ub");
+    const std::size_t N = static_cast<std::size_t>(c->N);
+    double* h = reinterpret_cast<double*>(stage(c, 2 * N * n * sizeof(double) + extra));
+    for(std::size_t a = 0; a < N && n; ++a) {
+        std::memcpy(h + a * n, lb + a * stride, n * sizeof(double));
+        std::memcpy(h + (N + a) * n, ub + a * stride, n * sizeof(double));
     }
-    std::vector<unsigned> d;
-    if(l.depth) {
-        d.assign(n, depth);
-        hip_check(hipMemcpyAsync(l.depth, d.data(), n * sizeof(unsigned), hipMemcpyHostToDevice, c->stream), "upload depth");
-    }
-    set_count(c, l.count, n);
-    sync(c);
+    launch(c, KIND_SET_COUNT, "k_load_boxes", [&] {
+        const unsigned blocks = static_cast<unsigned>(std::min<std::size_t>(2 * N * n / 256 + 1, 1024));
+        hipLaunchKernelGGL(k_load_boxes, dim3(blocks), dim3(256), 0, c->stream, l.view(), h, static_cast<unsigned long long>(n),
+                           static_cast<unsigned>(N), depth, c->d_state, whole ? 1u : 0u, c->segs);
+        return hipGetLastError();
+    });
 }
 void download_soa(sqd_core* c, const DevList& l, unsigned long long n, double* lb, double* ub, unsigned long long stride) {
     for(int a = 0; a < c->N; ++a) {
@@ -1042,14 +1088,7 @@ void prove_steps(sqd_core* c) {
     enum : unsigned { FIN = 1, SPL = 2, NEXT = 4 };
     auto run = [&](auto&& enqueue) {
         enqueue();
-        if(!c->h_done) {
-            enqueue_state_copy(c);
-            finish_state(c);
-            return;
-        }
-        const unsigned long long ticket = ++c->tickets;
-        enqueue_state_copy(c, ticket);
-        wait_done(c, ticket);
+        read_state(c);
     };
     if(c->ks->NSTAT == 0) {
         run([&] { enqueue_initial_queue(c); enqueue_round(c); });
@@ -1276,7 +1315,6 @@ void configure_core(sqd_core* c, int device, const sqd_program* program, const s
         c->undec_cap = undec_cap;
         lay.take(c->d_undec, static_cast<std::size_t>(undec_cap));
     }
-    lay.take(c->d_has, static_cast<std::size_t>(kmax));
     const std::size_t n_consts = 2 * static_cast<std::size_t>(std::max(1, c->ks->NC));
     lay.take(c->d_consts, n_consts);
     lay.take(c->d_box_ct, 2 * static_cast<std::size_t>(c->N));
@@ -1480,6 +1518,7 @@ void sqd_core_destroy(sqd_core* c) {
     if(c->stream) (void)hipStreamSynchronize(c->stream);
     if(c->d_jobs) (void)hipFree(c->d_jobs);
     if(c->h_state) (void)hipHostFree(c->h_state);
+    if(c->h_stage) (void)hipHostFree(c->h_stage);
     if(c->g_first) (void)hipGraphExecDestroy(c->g_first);
     if(c->g_round) (void)hipGraphExecDestroy(c->g_round);
     if(c->g_cont_start) (void)hipGraphExecDestroy(c->g_cont_start);
@@ -1524,35 +1563,33 @@ int sqd_nonfinal(sqd_core* c, const double* lb, const double* ub, size_t n,
         hip_check(hipSetDevice(c->device), "hipSetDevice");
         begin_call(c);
         check_groups_valid(c, lb, ub, n);
-        reset_state(c);
-        std::vector<double> clb, cub, hlb, hub;
-        for(std::size_t off = 0; off < n; off += c->k_max) {
+        // per chunk: the boxes in, the static levels, the hulls decoded straight
+        // into the staging memory, and one wait
+        const std::size_t N = static_cast<std::size_t>(c->N);
+        sqd_counts r{};
+        std::size_t off = 0;
+        do {
             const std::size_t m = std::min<std::size_t>(c->k_max, n - off);
-            clb.assign(static_cast<std::size_t>(c->N) * m, 0);
-            cub.assign(static_cast<std::size_t>(c->N) * m, 0);
-            for(int a = 0; a < c->N; ++a)
-                for(std::size_t i = 0; i < m; ++i) {
-                    clb[static_cast<std::size_t>(a) * m + i] = lb[static_cast<std::size_t>(a) * n + off + i];
-                    cub[static_cast<std::size_t>(a) * m + i] = ub[static_cast<std::size_t>(a) * n + off + i];
-                }
-            upload_soa(c, c->stack, clb.data(), cub.data(), m, 0);
-            levels_reset(c);
+            const std::size_t boxes = 2 * N * m * sizeof(double);
+            load_boxes(c, c->stack, lb ? lb + off : lb, ub ? ub + off : ub, m, n, 0, off == 0, boxes + m);
+            double* const hulls = reinterpret_cast<double*>(c->h_stage + boxes);
+            unsigned char* const has = reinterpret_cast<unsigned char*>(c->h_stage + 2 * boxes);
             if(c->ks->NSTAT > 0) run_static(c, dev::NONFINAL, c->stack.view(), nullptr, c->stack.count, m, c->crit.view());
             launch(c, KIND_HULL_DECODE, "decode", [&] {
-                return c->ks->hull_decode(c->stack.view(), m, c->d_hull, c->scratch.view(), c->d_has, c->stream);
+                dev::BoxList out{};
+                out.lb = hulls;
+                out.ub = hulls + N * m;
+                out.stride = m;
+                return c->ks->hull_decode(c->stack.view(), m, c->d_hull, out, has, c->stream);
             });
-            hlb.assign(static_cast<std::size_t>(c->N) * m, 0);
-            hub.assign(static_cast<std::size_t>(c->N) * m, 0);
-            download_soa(c, c->scratch, m, hlb.data(), hub.data(), m);
-            hip_check(hipMemcpyAsync(has_hull + off, c->d_has, m, hipMemcpyDeviceToHost, c->stream), "copy has");
-            sync(c);
-            for(int a = 0; a < c->N; ++a)
-                for(std::size_t i = 0; i < m; ++i) {
-                    hull_lb[static_cast<std::size_t>(a) * n + off + i] = hlb[static_cast<std::size_t>(a) * m + i];
-                    hull_ub[static_cast<std::size_t>(a) * n + off + i] = hub[static_cast<std::size_t>(a) * m + i];
-                }
-        }
-        sqd_counts r = counts_of(read_state(c));
+            r = counts_of(read_state(c));
+            for(std::size_t a = 0; a < N && m; ++a) {
+                std::memcpy(hull_lb + a * n + off, hulls + a * m, m * sizeof(double));
+                std::memcpy(hull_ub + a * n + off, hulls + (N + a) * m, m * sizeof(double));
+            }
+            if(m) std::memcpy(has_hull + off, has, m);
+            off += m;
+        } while(off < n);
         end_call(c);
         if(c->ks->NSTAT == 0) r.num_leaf_cuboids += n;  // without static variables each box is its own leaf
         if(counts) *counts = r;
@@ -1567,8 +1604,7 @@ int sqd_final(sqd_core* c, const double* lb, const double* ub, size_t n,
         if(n > c->fin.cap) throw Failure(SQD_ERR_CAPACITY, "too many boxes for one final pass");
         begin_call(c);
         check_groups_valid(c, lb, ub, n);
-        reset_state(c);
-        upload_soa(c, c->fin, lb, ub, n, 0);
+        load_boxes(c, c->fin, lb, ub, n, n, 0, true);
         if(c->ks->NSTAT > 0) run_static(c, dev::FINAL, c->fin.view(), nullptr, c->fin.count, n, c->crit.view());
         else launch(c, KIND_FINAL_NOSTATIC, "final", [&] {
             return c->ks->final_nostatic(c->fin.view(), c->crit.view(), c->d_slots,
@@ -1599,8 +1635,7 @@ int sqd_split(sqd_core* c, const double* lb, const double* ub, size_t n,
         hip_check(hipSetDevice(c->device), "hipSetDevice");
         if(n > c->spl.cap) throw Failure(SQD_ERR_CAPACITY, "too many boxes for one split");
         begin_call(c);
-        reset_state(c);
-        upload_soa(c, c->spl, lb, ub, n, 1);
+        load_boxes(c, c->spl, lb, ub, n, n, 1, true);
         run_dynamic(c, dev::SPLIT, c->spl.view(), c->spl.count, n, c->stack.view());
         const DeviceState& h = read_state(c);
         const unsigned long long k = h.stack_count;
