@@ -26,7 +26,7 @@
 //   deps(list, f)            calls f(a) for each bound index a in update list `list`
 //   rows_violated<L>(lb, ub, C)   constraint rows of static level L
 //   all_satisfied(lb, ub, C)      every remaining constraint possibly holds
-//   level_waves(L), prop_fast(L)  per-level register budget and propagation form
+//   level_waves(L), prop_fast(L)  per-level register budget (0: the default) and propagation form
 #pragma once
 #include <type_traits>
 #include "interval.hpp"
@@ -47,10 +47,13 @@ constexpr int kBlock = 256;
 #define SQD_LEVEL_ATTR
 #endif
 // The binary64 static level kernels take their program's budget for the level
-// (P::level_waves(L); 0 or 1: no minimum) unless SQD_LEVEL_WAVES_PER_EU is set.
+// (P::level_waves(L)) or else 3 waves, unless SQD_LEVEL_WAVES_PER_EU is set.  3
+// waves allow 168 VGPRs: Four's level 1 (180 and 2 waves left to the compiler) 305
+// -> 242 us for 3.3 M children without a spill, the levels that needed less
+// unchanged; 4 waves made More2's level 1 214 -> 262 us.
 template<class P, int L>
 constexpr int static_level_waves() {
-    return SQD_LEVEL_WAVES_PER_EU > 0 ? SQD_LEVEL_WAVES_PER_EU : (P::level_waves(L) > 0 ? P::level_waves(L) : 1);
+    return SQD_LEVEL_WAVES_PER_EU > 0 ? SQD_LEVEL_WAVES_PER_EU : (P::level_waves(L) > 0 ? P::level_waves(L) : 3);
 }
 
 // The kernel with the group test holds both the test and the per-child decision;

@@ -539,7 +539,7 @@ std::string generate(const flat::Program& p, const std::string& key) {
     table("st_arg", sta, [](const flat::FSplit& s) { return s.arg; });
     table("st_subs", sta, [](const flat::FSplit& s) { return static_cast<int>(s.subs); });
     // Register budget of the per-child binary64 level kernels (k_static_level) as
-    // resident waves per SIMD (0: the compiler's choice).  On a last level that is
+    // resident waves per SIMD (0: the kernels' default).  On a last level that is
     // the pass over the children binary32 left undecided; the values were measured
     // on whole levels decided child by child: One's and Two's level 1 at 4 (128
     // VGPRs, a few spilled; 3 was slower), Three's level 1 at 4 (274 against 292
