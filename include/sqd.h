@@ -82,8 +82,9 @@ typedef struct sqd_settings {
                                       in binary64 with the group test: the rows are first
                                       checked once per group of prefilter_group consecutive
                                       children, the children of the groups left one by one;
-                                      exactly the results of the plain pass (no counterpart in
-                                      the reference; levels in fp32_prefilter take that) */
+                                      exactly the results of deciding every child by itself (no
+                                      counterpart in the reference; levels in fp32_prefilter take
+                                      that; the last level does it without being asked) */
 } sqd_settings;
 
 #define SQD_FP32_ALL_LEVELS 0xffffffffu

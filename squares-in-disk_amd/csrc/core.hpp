@@ -49,7 +49,7 @@ constexpr int kBlock = 256;
 // The binary64 static level kernels take their program's budget for the level
 // (P::level_waves(L)) or else 3 waves, unless SQD_LEVEL_WAVES_PER_EU is set.  3
 // waves allow 168 VGPRs: Four's level 1 (180 and 2 waves left to the compiler) 305
-// -> 242 us for 3.3 M children without a spill, the levels that needed less
+// -> 242 us for 3.3 M children (48 bytes of scratch), the levels that needed less
 // unchanged; 4 waves made More2's level 1 214 -> 262 us.
 template<class P, int L>
 constexpr int static_level_waves() {
@@ -67,7 +67,7 @@ enum Mode : int { NONFINAL = 0, FINAL = 1, SPLIT = 2, INIT = 3 };
 struct NoHoist {};
 // Flag or'ed into a static-level mode at launch: the FP32-prefiltered kernel.
 constexpr int kModeF32 = 4;
-// Static-level mode bit: binary64 with the group test (k_static_group64).
+// Static-level mode bit: binary64 with the group test (k_static_grouped).
 constexpr int kModeGroup = 8;
 
 struct DeviceCounters {
@@ -329,17 +329,6 @@ __device__ __forceinline__ unsigned long long wave_append(bool flag, unsigned lo
     base = __shfl(base, first);
     return base + static_cast<unsigned long long>(__popcll(mask & ((1ull << lane) - 1ull)));
 }
-// The same with n entries for every flagged lane (n equal on all lanes).
-__device__ __forceinline__ unsigned long long wave_append_n(bool flag, unsigned n, unsigned long long* counter) {
-    const unsigned long long mask = __ballot(flag);
-    const unsigned long long active = __ballot(1);
-    const int lane = __lane_id();
-    const int first = __ffsll(static_cast<long long>(active)) - 1;
-    unsigned long long base = 0;
-    if(lane == first && mask) base = atomicAdd(counter, static_cast<unsigned long long>(__popcll(mask)) * n);
-    base = __shfl(base, first);
-    return base + static_cast<unsigned long long>(__popcll(mask & ((1ull << lane) - 1ull))) * n;
-}
 __device__ __forceinline__ unsigned long long wave_sum(unsigned long long v) {
 #pragma unroll
     for(int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
@@ -387,14 +376,6 @@ __device__ __forceinline__ void load_consts_f32(float* dst, const double* src) {
     __syncthreads();
 }
 
-// A value equal on every lane of the wave, held in scalar registers from here
-// on (the compiler cannot tell that a value loaded from memory or derived from
-// threadIdx.x / 64 is the same on all lanes, and keeps it in vector registers).
-__device__ __forceinline__ unsigned long long wave_uniform(unsigned long long v) {
-    const unsigned lo = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(v));
-    const unsigned hi = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(v >> 32));
-    return (static_cast<unsigned long long>(hi) << 32) | lo;
-}
 // The inputs of a level: n of them, numbered segment by segment where the list is
 // segmented.  Counts are clamped to the list's (or segment's) capacity (a count
 // past it was raised by a pass that could not store its survivors, which set the
