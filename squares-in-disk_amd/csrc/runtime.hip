@@ -202,10 +202,13 @@ __global__ __launch_bounds__(kEndThreads) void k_round_end(DeviceState* st, unsi
     if(w < kStateWords && out) __hip_atomic_store(out + w, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     if(w >= kKeptWords && w < kStateWords) words[w] = 0ull;
     if(done) {
-        // tells a host that polls that its copy of the job's state is complete: the
-        // barrier waits for the stores above, which go past the caches to the
-        // (coherent) host memory; a system fence would write back the whole L2,
-        // 8 us where a level left its list there
+        // tells a host that polls that its copy of the job's state is complete.  The
+        // state's stores go past the caches to the (coherent) host memory, and every
+        // wave waits until its own are acknowledged there: the barrier orders memory
+        // inside the block only, and would let the ticket overtake them.  (A system
+        // fence would write back the whole L2 as well, 8 us where a level left its
+        // list there.)
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
         if(w == 0) __hip_atomic_store(done + blockIdx.y, ticket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
