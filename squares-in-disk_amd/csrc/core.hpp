@@ -1292,8 +1292,16 @@ __global__ __launch_bounds__(kBlock) void k_round_nostatic(BoxList stack, RoundW
     block_counts_add(block_counts, 0ull, c_leaf, c_crit);
 }
 
-// Decode hull records in input order (sqd_nonfinal): entry d of `out` holds the
-// hull of input d, has[d] = 0 when no leaf survived.
+// Stores to pinned host memory that the host reads without waiting for the kernel's
+// end (it polls a ticket that a later store or kernel writes): past the caches, and
+// acknowledged there when host_stores_done() returns.
+template<class T> __device__ __forceinline__ void host_store(T* p, T v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+__device__ __forceinline__ void host_stores_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+// Decode hull records in input order (sqd_nonfinal): entry d of `out` (in pinned
+// host memory, as `has`) holds the hull of input d, has[d] = 0 when no leaf survived.
 template<class P>
 __global__ __launch_bounds__(kBlock) void k_hull_decode(BoxList items, unsigned long long n, unsigned long long* hull,
                                                         BoxList out, unsigned char* has) {
@@ -1317,8 +1325,13 @@ __global__ __launch_bounds__(kBlock) void k_hull_decode(BoxList items, unsigned 
         }
         if(ok) clear_hull_record(rec, N);
     }
-    store_box<P>(out, d, lb, ub);
-    has[d] = ok ? 1 : 0;
+#pragma unroll
+    for(int a = 0; a < N; ++a) {
+        host_store(reinterpret_cast<std::uint64_t*>(out.lb) + a * out.stride + d, bits(lb[a]));
+        host_store(reinterpret_cast<std::uint64_t*>(out.ub) + a * out.stride + d, bits(ub[a]));
+    }
+    host_store(has + d, static_cast<unsigned char>(ok ? 1 : 0));
+    host_stores_done();
 }
 
 // Final pass without static variables outside a round: every cuboid is one critical leaf.  Row

@@ -199,7 +199,7 @@ __global__ __launch_bounds__(kEndThreads) void k_round_end(DeviceState* st, unsi
         for(unsigned k = 0; k < kEndThreads / 64; ++k) v += part[w < 3 ? w : w - 1][k];
         words[w] = v;
     }
-    if(w < kStateWords && out) __hip_atomic_store(out + w, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if(w < kStateWords && out) dev::host_store(out + w, v);
     if(w >= kKeptWords && w < kStateWords) words[w] = 0ull;
     if(done) {
         // tells a host that polls that its copy of the job's state is complete.  The
@@ -208,9 +208,9 @@ __global__ __launch_bounds__(kEndThreads) void k_round_end(DeviceState* st, unsi
         // inside the block only, and would let the ticket overtake them.  (A system
         // fence would write back the whole L2 as well, 8 us where a level left its
         // list there.)
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        dev::host_stores_done();
         __syncthreads();
-        if(w == 0) __hip_atomic_store(done + blockIdx.y, ticket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        if(w == 0) dev::host_store(done + blockIdx.y, ticket);
     }
 }
 // Boxes that a caller hands over, from pinned host memory (N * n lower, then N * n

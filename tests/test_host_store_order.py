@@ -45,3 +45,17 @@ def test_state_before_ticket(tmp_path):
     # every wave passes the wait: it stands in the barrier's own basic block
     block = max(i for i, l in enumerate(code[:barrier]) if l.endswith(":") or l.startswith("s_cbranch"))
     assert any(_waits(l) for l in code[max(block, host[-2]):barrier])
+
+
+def test_hulls_before_the_kernel_ends(tmp_path):
+    # the hulls are announced by the ticket of a later kernel: they have to be out
+    # (past the caches, and acknowledged) when this one ends
+    code = _kernel(build.GEN / "ec2.hip", "k_hull_decode", tmp_path)
+    stores = [i for i, l in enumerate(code) if l.startswith(("global_store", "flat_store"))]
+    host = [i for i in stores if "sc0 sc1" in code[i]]
+    assert len(host) == 2 * 4 + 1                                  # two bounds of four variables, and `has`
+    end = code.index("s_endpgm")
+    # the wait follows the stores in their own basic block: no lane that stored skips it
+    block = [l for l in code[host[-1]:end]]
+    wait = next(i for i, l in enumerate(block) if _waits(l))
+    assert not any(l.endswith(":") or l.startswith("s_cbranch") for l in block[:wait])
