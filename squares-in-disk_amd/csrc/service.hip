@@ -317,6 +317,11 @@ struct sqd_service {
     // it), destroying idle cores of other programs or waiting as needed.
     // Returns the slot id, 0 when the service stops.
     uint64_t acquire(std::unique_lock<std::mutex>& lk, const sqd_program* prog) {
+        struct Wanted {                       // this worker's part of room_wanted
+            sqd_service* s;
+            bool on = false;
+            ~Wanted() { if(on) --s->room_wanted; }
+        } wanted{this};
         for(;;) {
             if(stop) return 0;
             for(auto& s : pool)
@@ -345,12 +350,16 @@ struct sqd_service {
                     freed = true;
                     break;
                 }
-            if(!freed) {
+            if(freed) continue;
+            // open batches without jobs give up their cores: told once, when the
+            // worker starts to want room (told at each wake-up, two workers here
+            // would wake each other until a core is free)
+            if(!wanted.on) {
+                wanted.on = true;
                 ++room_wanted;
-                cv.notify_all();   // open batches without jobs give up their cores
-                cv.wait(lk);
-                --room_wanted;
+                cv.notify_all();
             }
+            cv.wait(lk);
         }
     }
 
