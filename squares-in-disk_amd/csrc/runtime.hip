@@ -1028,7 +1028,8 @@ void drain_criticals(sqd_core* c, unsigned long long k, unsigned long long n_fin
             std::vector<unsigned long long> n(static_cast<std::size_t>(src.segs - 1) * dev::kSegStride + 1);
             hip_check(hipMemcpyAsync(n.data(), src.count, n.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost,
                                      c->stream), "copy segment counters");
-            read_state(c);
+            enqueue_state_copy(c);
+            finish_state(c);   // waits for the stream: the copy above ends with it, not with a ticket
             ranges.clear();
             for(unsigned g = 0; g < src.segs; ++g)
                 ranges.push_back({g * src.seg_cap, std::min(n[static_cast<std::size_t>(g) * dev::kSegStride], src.seg_cap)});
