@@ -1215,9 +1215,9 @@ void prove_jobs(sqd_core* c, unsigned n, const uint32_t* first, const uint32_t* 
 // of `program` on `device` (nothing is allocated): the sizes follow from the
 // settings, and the rounds are bounded so that no level list and no undecided
 // list can overflow.  `state_words` receives the place of the control block in
-// the layout.
+// the layout; without `segments` every level list is dense.
 void configure_core(sqd_core* c, int device, const sqd_program* program, const sqd_settings* settings, Layout& lay,
-                    unsigned long long*& state_words) {
+                    unsigned long long*& state_words, bool segments = true) {
     if(!program->ks)
         throw Failure(SQD_ERR_NO_KERNELS, "no kernels are compiled for this program (fingerprint not registered)");
     c->device = device;
@@ -1255,10 +1255,15 @@ void configure_core(sqd_core* c, int device, const sqd_program* program, const s
     if(worst_init > lvl_cap) throw Failure(SQD_ERR_CAPACITY, "initial queue levels do not fit the level buffers");
     c->split_fanout = product(c->dyn_subs, c->dyn_subs.size());
     unsigned long long kmax = s.dequeue_buffer_size ? s.dequeue_buffer_size : 8192;
-    // Level lists in segments (dev::BoxList): a segment receives at most its
-    // share of a level's children and two waves more, so the lists keep that
-    // much room; buffers too small for it hold dense lists.  The counters come
-    // out of the level buffers' bytes.
+    kmax = std::min(kmax, lvl_cap / worst_static);
+    kmax = std::min(kmax, lvl_cap / worst_split);
+    // Level lists in segments (dev::BoxList): a segment receives at most its share
+    // of a level's children and two waves more.  That slack and the counters come on
+    // top of level_bytes (for One 250 KB and 8 KB per job), so that a round and a
+    // host-driven call take as many cuboids as with dense lists.  Lists that the
+    // slack would lengthen by more than a quarter stay dense: their levels append at
+    // most 128 waves on one counter, 1.5 us (1,152 with a group test before the
+    // last level, 14 us).
     unsigned n_lists = 0;
     for(int mode : {dev::NONFINAL, dev::FINAL})
         for(std::size_t L = 0; L + 1 < c->st_subs.size() && n_lists < sizeof(SegIndex); ++L)
@@ -1271,17 +1276,11 @@ void configure_core(sqd_core* c, int device, const sqd_program* program, const s
     // place of their parents, which evens out only within each input segment)
     const unsigned before_last = used >> 1;
     const unsigned long long slack = 64ull * dev::kSegs * ((s.group_levels & before_last) ? dev::kSegs + 2 : 2);
-    const unsigned long long counter_entries = (counter_words * sizeof(unsigned long long) + 512 + per_entry - 1) / per_entry;
-    unsigned long long room = lvl_cap;   // entries the rounds may fill
-    if(n_lists > 0 && lvl_cap < (1ull << 32) && lvl_cap > counter_entries + slack &&
-       (lvl_cap - counter_entries - slack) / std::max(worst_static, worst_split) >= 1 &&
-       lvl_cap - counter_entries - slack >= worst_init) {
+    const unsigned long long room = lvl_cap;   // entries the rounds may fill
+    if(segments && n_lists > 0 && lvl_cap + slack < (1ull << 32) && lvl_cap >= 4 * slack) {
         c->segs.n_lists = n_lists;
-        lvl_cap -= counter_entries;
-        room = lvl_cap - slack;
+        lvl_cap += slack;
     }
-    kmax = std::min(kmax, room / worst_static);
-    kmax = std::min(kmax, room / worst_split);
     // the FP32 prefilter lists the children it leaves undecided (8 bytes each,
     // level_bytes of them), up to all children of the level, so a round is bounded
     // by the largest such level's children per dynamic cuboid
@@ -2009,10 +2008,18 @@ int sqd_prove_range_noalloc(int device, const sqd_program* program, const sqd_se
         else sqd_settings_default(&s);
         s.jobs = 1;     // one job's layout
         s.graphs = 0;   // a graph would be an allocation
-        sqd_core c;     // host-side state only; its stream is the device's null stream
+        // host-side state only; its stream is the device's null stream.  Dense level
+        // lists where the segments' slack does not fit the array.
+        auto core = std::make_unique<sqd_core>();
         Layout lay;
         unsigned long long* state_words = nullptr;
-        configure_core(&c, device, program, &s, lay, state_words);
+        configure_core(core.get(), device, program, &s, lay, state_words);
+        if(core->job_stride > kScratchBytes && core->segs.n_lists) {
+            core = std::make_unique<sqd_core>();
+            lay = Layout();
+            configure_core(core.get(), device, program, &s, lay, state_words, false);
+        }
+        sqd_core& c = *core;
         if(c.job_stride > kScratchBytes)
             throw Failure(SQD_ERR_CAPACITY, "these settings need " + std::to_string(c.job_stride) +
                                                 " bytes of device memory, the scratch array of sqd_prove_range_noalloc "
