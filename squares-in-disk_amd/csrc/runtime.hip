@@ -396,7 +396,7 @@ struct sqd_core {
     void* progress_user = nullptr;
     double progress_start = 0, progress_every = 0;
     std::vector<double> head;        // 2N: the frontier's top for progress reports
-    bool groups_valid = true;        // the current call's boxes allow the binary64 group test
+    bool groups_valid = true;        // the current call's boxes allow the group tests and the prefilter
     bool fp32 = false;               // some static level runs the FP32-prefiltered kernels
     // sqd_prove as HIP graphs: the initial queue with the first round, and one later round
     hipGraphExec_t g_first = nullptr, g_round = nullptr;
@@ -678,11 +678,11 @@ void run_static_level(sqd_core* c, int mode, int L, const dev::BoxList& in, cons
     if(count == &c->d_state->round.round_k) a.pop = &c->d_state->round;   // a round's first level takes its cuboids
     a.undec_count = &c->d_state->undec_count[mode * 16 + L];
     // the group test: sized by the settings on the levels that ask for one (here or
-    // in the prefilter), by the kernel on the last level of a plain proof; off
-    // (one child per group) for boxes it is not valid for
+    // in the prefilter), by the kernel on the last level of a plain proof.  Boxes that
+    // the tests are not valid for take neither: binary64, one child per group
     const bool asked = ((c->settings.fp32_prefilter | c->settings.group_levels) >> L) & 1u;
-    const bool f32 = (c->settings.fp32_prefilter >> L) & 1u;
-    if(!f32 && !c->groups_valid) a.children_per_lane = 1;
+    const bool f32 = c->groups_valid && ((c->settings.fp32_prefilter >> L) & 1u);
+    if(!c->groups_valid) a.children_per_lane = 1;
     else if(!asked) a.children_per_lane = 0;
     const unsigned long long children = max_items * c->st_subs[static_cast<std::size_t>(L)];
     launch(c, mode * 16 + L, "static level launch",
@@ -811,10 +811,11 @@ void begin_call(sqd_core* c) {
     }
     c->clean = 0;   // until the call completes
 }
-// The group test decides like the per-child test where the interval operations
-// are inclusion-isotone: on finite boxes inside the program's compile-time box,
-// whose signs the generated code relies on.  Boxes of a proof always are; for
-// boxes (SoA, stride n) that a caller hands over, this is checked.
+// The group tests and the binary32 prefilter decide like the per-child binary64
+// test where the interval operations are inclusion-isotone: on finite boxes inside
+// the program's compile-time box, whose signs the generated code relies on.  Boxes
+// of a proof always are; for boxes (SoA, stride n) that a caller hands over, this is
+// checked.
 void check_groups_valid(sqd_core* c, const double* lb, const double* ub, std::size_t n) {
     const auto& prog = c->program->prog;
     bool ok = true;

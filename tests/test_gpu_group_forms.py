@@ -1,0 +1,70 @@
+"""The group tests where groups really form: with one or three blocks per launch the
+children of a level take many trips, so that the first test runs, its groups are
+split, listed, left untested and decided in ragged waves.  Decisions, hulls and
+criticals are the oracle's bit for bit (it decides every child by itself), so no
+tolerance is involved."""
+import numpy as np
+import pytest
+
+import pyoracle
+import sqd
+
+pytestmark = pytest.mark.gpu
+
+ALL = 0xFFFFFFFF
+
+
+def _bits(a):
+    return np.ascontiguousarray(a, dtype=np.float64).view(np.uint64)
+
+
+def _rows(lb, ub):
+    m = np.empty((lb.shape[1], 2 * lb.shape[0]), dtype=np.uint64)
+    m[:, 0::2], m[:, 1::2] = _bits(lb).T, _bits(ub).T
+    return m[np.lexsort(m.T[::-1])]
+
+
+def _core(key, **kw):
+    return sqd.Core(sqd.Program.from_lemma(key), settings=sqd.default_settings(level_bytes=64 << 20, frontier_capacity=1 << 16, **kw))
+
+
+def _queue(program_text, key, count):
+    o = pyoracle.Oracle(program_text(key))
+    lb, ub, _ = o.initial_queue()
+    at = np.linspace(0, lb.shape[1] - 1, min(count, lb.shape[1])).astype(int)
+    return o, lb[:, at], ub[:, at]
+
+
+def _same_nonfinal(want, got):
+    ohl, ohu, ohas, oc = want
+    ghl, ghu, ghas, gc = got
+    assert gc["num_cuboids"] == oc["num_cuboids"] and gc["num_leaf_cuboids"] == oc["num_leaf_cuboids"]
+    assert np.array_equal(ghas, ohas)
+    keep = ohas.astype(bool)
+    assert np.array_equal(_bits(ghl[:, keep]), _bits(ohl[:, keep]))
+    assert np.array_equal(_bits(ghu[:, keep]), _bits(ohu[:, keep]))
+
+
+def _same_final(want, got):
+    assert got[2] == want[2]
+    assert np.array_equal(_rows(got[0], got[1]), _rows(want[0], want[1]))
+
+
+# More2's fifth variable 6 below its domain (moved there, or widened): a group's
+# interval can then miss values of its children, so that the group tests would prune
+# children that are not to be pruned
+@pytest.mark.parametrize("widen", [False, True])
+@pytest.mark.parametrize("kw", [{}, {"group_levels": ALL, "prefilter_group": 16},
+                                {"fp32_prefilter": ALL, "prefilter_group": 16}], ids=["plain", "group", "fp32"])
+def test_boxes_outside_the_domain(program_text, widen, kw):
+    o, lb, ub = _queue(program_text, "more2", 24)
+    lb[4] -= 6.0
+    if not widen:
+        ub[4] -= 6.0
+    with _core("more2", grid_blocks=1, **kw) as core:
+        _same_nonfinal(o.nonfinal(lb, ub), core.nonfinal(lb, ub))
+        _same_final(o.final(lb, ub), core.final(lb, ub))
+        # a call with boxes of the domain has its group tests again
+        _, lb, ub = _queue(program_text, "more2", 5)
+        if "fp32_prefilter" not in kw:
+            _same_nonfinal(o.nonfinal(lb, ub), core.nonfinal(lb, ub))
