@@ -50,6 +50,50 @@ def _same_final(want, got):
     assert np.array_equal(_rows(got[0], got[1]), _rows(want[0], want[1]))
 
 
+@pytest.mark.parametrize("key,count", [("one", 7), ("two", 13), ("three", 33), ("four", 3), ("more1", 3), ("more2", 3),
+                                       ("ec2", 15), ("ec3", 3)])
+def test_plain_nonfinal(program_text, key, count):
+    o, lb, ub = _queue(program_text, key, count)
+    want = o.nonfinal(lb, ub)
+    for blocks in (1, 3):
+        with _core(key, grid_blocks=blocks) as core:
+            _same_nonfinal(want, core.nonfinal(lb, ub))
+
+
+@pytest.mark.parametrize("key,count", [("two", 13), ("four", 3), ("ec2", 15), ("ec3", 3)])
+@pytest.mark.parametrize("group", [0, 1, 2, 8, 16, 32, 64])
+def test_every_level_grouped(program_text, key, count, group):
+    o, lb, ub = _queue(program_text, key, count)
+    with _core(key, grid_blocks=1, group_levels=ALL, prefilter_group=group) as core:
+        _same_nonfinal(o.nonfinal(lb, ub), core.nonfinal(lb, ub))
+
+
+def _pieces(lb, ub, m):
+    """Each box cut into m along the first variable."""
+    lb, ub = np.repeat(lb, m, axis=1), np.repeat(ub, m, axis=1)
+    j = np.tile(np.arange(m), lb.shape[1] // m)
+    w = (ub[0] - lb[0]) / m
+    lb[0], ub[0] = lb[0] + w * j, lb[0] + w * (j + 1)
+    return lb, ub
+
+
+# ec2's last level has 64 children of a box, ec3's 128 (8 of the first level's each):
+# groups that fail as a whole, in part and not at all, and real criticals
+@pytest.mark.parametrize("key,pieces", [("ec2", 5), ("ec2", 37), ("ec3", 1), ("ec3", 9)])
+@pytest.mark.parametrize("kw", [{}, {"prefilter_group": 2}, {"prefilter_group": 8}, {"prefilter_group": 16},
+                                {"prefilter_group": 32}, {"prefilter_group": 64}], ids=lambda k: str(list(k.values())))
+def test_final_criticals(program_text, key, pieces, kw):
+    o, lb, ub = _queue(program_text, key, 16)
+    lb, ub = _pieces(lb, ub, pieces)
+    want = o.final(lb, ub)
+    assert 0 < want[2]["num_critical_cuboids"] < want[2]["num_leaf_cuboids"] or key == "ec2"
+    if kw:
+        kw = dict(kw, group_levels=ALL)
+    for blocks in (1, 2):
+        with _core(key, grid_blocks=blocks, **kw) as core:
+            _same_final(want, core.final(lb, ub))
+
+
 # More2's fifth variable 6 below its domain (moved there, or widened): a group's
 # interval can then miss values of its children, so that the group tests would prune
 # children that are not to be pruned
