@@ -69,6 +69,8 @@ struct Emitter {
     // nodes whose values are read from the hoisted-term struct `h` instead of
     // being computed (set while emitting a level's hoisted row check)
     std::set<int> subst;
+    // nodes whose value has to be the exact one everywhere (exact_nodes)
+    std::vector<char> exact;
 
     void collect(int id, std::vector<int>& order, std::vector<char>& seen) {
         if(seen[static_cast<std::size_t>(id)]) return;
@@ -255,7 +257,8 @@ struct Emitter {
                 // domain checks only where the compile-time bounds leave [-1, 1]
                 const bool chk_lb = KN(0).lb < fpb::int_to_fp(-1), chk_ub = KN(0).ub > fpb::int_to_fp(1);
                 o << "const IV " << v(id) << " = iv_acos<" << (chk_lb ? "true" : "false") << ", "
-                  << (chk_ub ? "true" : "false") << ", EXACT>(" << v(K(0)) << ");";
+                  << (chk_ub ? "true" : "false") << ", " << (exact[static_cast<std::size_t>(id)] ? "true" : "EXACT") << ">("
+                  << v(K(0)) << ");";
                 break;
             }
             case FOp::BoolConst: o << "const IB " << b(id) << "{" << (n.b_def ? "true" : "false") << ", " << (n.b_poss ? "true" : "false") << "};"; break;
@@ -271,12 +274,28 @@ struct Emitter {
     }
 };
 
+// Nodes that something reads whose code relies on compile-time bounds: products,
+// quotients and square roots drop the sign cases that the bounds exclude, and an arc
+// cosine the domain checks.  A wider interval there can cross such a bound, and the
+// operation then gives one that does not contain the exact result.  (Sums, minima,
+// squares, conditionals, comparisons and connectives hold for any interval.)
+std::vector<char> exact_nodes(const Program& p) {
+    std::vector<char> exact(p.nodes.size(), 0);
+    for(std::size_t i = p.nodes.size(); i-- > 0;) {   // readers have higher ids
+        const FOp op = p.nodes[i].op;
+        const bool relies = op == FOp::Mul || op == FOp::Div || op == FOp::Sqrt || op == FOp::Acos;
+        if(!relies && !exact[i]) continue;
+        for(int k : p.nodes[i].kids) exact[static_cast<std::size_t>(k)] = 1;
+    }
+    return exact;
+}
+
 } // namespace
 
 bool supported(const flat::Program&) { return true; }
 
 std::string generate(const flat::Program& p, const std::string& key) {
-    Emitter e{p, {}, {}};
+    Emitter e{p, {}, {}, {}, exact_nodes(p)};
     const std::string ns = "sqd_gen_" + key;
     std::vector<int> dyn, sta;
     for(std::size_t i = 0; i < p.splits.size(); ++i) (p.splits[i].dynamic ? dyn : sta).push_back(static_cast<int>(i));
@@ -286,14 +305,15 @@ std::string generate(const flat::Program& p, const std::string& key) {
     // correctly rounded arc cosines of the reference; with EXACT = false they are
     // the cheap enclosures (some 40 operations instead of thousands), whose
     // intervals contain the exact ones: a constraint that fails with them fails
-    // exactly too, so the checks below try it first.
-    std::vector<char> acos_dep(p.nodes.size(), 0);   // nodes that read an arc cosine
+    // exactly too, so the checks below try it first.  Arc cosines whose exact value
+    // is needed (exact_nodes) are exact either way.
+    std::vector<char> acos_dep(p.nodes.size(), 0);   // nodes that read an enclosed arc cosine
     for(std::size_t i = 0; i < p.nodes.size(); ++i) {
-        acos_dep[i] = p.nodes[i].op == FOp::Acos;
+        acos_dep[i] = p.nodes[i].op == FOp::Acos && !e.exact[i];
         for(int k : p.nodes[i].kids) acos_dep[i] = acos_dep[i] || acos_dep[static_cast<std::size_t>(k)];
     }
     // the checks `if(!c(...).poss) <fail>` of a list of constraints: all with
-    // enclosures, then those that read an arc cosine again with the exact values
+    // enclosures, then those that read an enclosed arc cosine again with the exact values
     // (in binary32 the enclosures are all there is)
     auto checks = [&](std::ostringstream& o, const std::vector<int>& list, const std::string& indent, const std::string& fail) {
         for(int c : list) o << indent << "if(!c" << c << "<false>(lb, ub, C).poss) " << fail << "\n";
