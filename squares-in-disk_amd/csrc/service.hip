@@ -291,7 +291,11 @@ struct sqd_service {
     uint64_t frontier_in_flight = 0;
     std::map<const sqd_program*, double> frontier_per_unit;
     sqd_service_stats stats{};
-    // how long a batch without jobs stays open, and the workers waiting for memory
+    // How long a batch without jobs stays open, and the workers waiting for memory.
+    // A client that hands over a program's jobs some milliseconds apart finds the
+    // batch open as it did when a proof took that long; it is neither faster nor
+    // slower so (jobs one after the other, open 20 ms against closed at once: Top2
+    // 60.6 and 58.7 us, One 86.3 and 85.6, One, Three and Six in turn 258 and 257).
     static constexpr std::chrono::milliseconds kBatchOpen{20};
     unsigned room_wanted = 0;
     bool stop = false;

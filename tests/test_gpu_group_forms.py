@@ -112,3 +112,17 @@ def test_boxes_outside_the_domain(program_text, widen, kw):
         _, lb, ub = _queue(program_text, "more2", 5)
         if "fp32_prefilter" not in kw:
             _same_nonfinal(o.nonfinal(lb, ub), core.nonfinal(lb, ub))
+
+
+@pytest.mark.parametrize("key,var", [("three", 0), ("three", 4), ("more1", 0), ("more1", 2)])
+@pytest.mark.parametrize("how", ["inverted", "infinite"])
+def test_inverted_and_infinite_boxes(program_text, key, var, how):
+    o, lb, ub = _queue(program_text, key, 6)
+    if how == "inverted":
+        lb[var], ub[var] = ub[var].copy(), lb[var].copy()
+    else:
+        ub[var] = np.inf
+    with _core(key, grid_blocks=1) as core:
+        _same_nonfinal(o.nonfinal(lb, ub), core.nonfinal(lb, ub))
+        _same_final(o.final(lb, ub), core.final(lb, ub))
+        _same_final(o.split(lb, ub), core.split(lb, ub))
