@@ -429,7 +429,8 @@ int sqd_service_get_stats(sqd_service* service, sqd_service_stats* out);
  * (its ProofInformation, ivarp/include/ivarp/prover/proof_information.hpp,
  * holds counts only); used by the throughput measurement. */
 typedef struct sqd_kernel_stat {
-    char name[48];        /* "static_level<NONFINAL,1>", "hull_finalize", ... */
+    char name[48];        /* "static_level<NONFINAL,0>", "static_level_group64<NONFINAL,1>" (with the
+                             group test), "static_level_fp32<...>", "hull_finalize", ... */
     int32_t mode;         /* 0 non-final, 1 final, 2 split, 3 initial queue, -1 other kernels */
     int32_t level;        /* static or dynamic level; -1 for other kernels */
     uint64_t launches;

@@ -112,15 +112,14 @@ struct RoundWords {
 };
 // Start of a proof, done by the first kernel of the initial queue (one block per
 // job): n_words words at `words` (the control block) and the counters of the
-// segmented lists to zero, the job's range from host memory to `range`, and the
-// box (N lb, N ub) as the level's only input.  With `flagged` only the jobs whose
-// start flag is set start; the others get no input.
+// segmented lists to zero, the job's range from host memory, and the box (N lb, N
+// ub) as the level's only input.  With `flagged` only the jobs whose start flag is
+// set start; the others get no input.
 struct StartArgs {
     unsigned long long* words;        // nullptr: no start (the input list is used)
     unsigned n_words;
     const double* box;
     const unsigned* host_ranges;      // pinned: lo[64], hi[64], start[64]
-    unsigned long long* range;        // first, last, start flag
     unsigned flagged;
     unsigned long long* seg_counters;
     unsigned seg_lists;

@@ -398,7 +398,7 @@ struct sqd_core {
     std::vector<double> head;        // 2N: the frontier's top for progress reports
     bool groups_valid = true;        // the current call's boxes allow the group tests and the prefilter
     bool fp32 = false;               // some static level runs the FP32-prefiltered kernels
-    // sqd_prove as HIP graphs: the initial queue with the first round, and one later round
+    // whole rounds of a proof as HIP graphs: the initial queue with the first round, and one later round
     hipGraphExec_t g_first = nullptr, g_round = nullptr;
     // continuous batches (sqd_batch_admit / sqd_batch_step): per row 0 free, 1 admitted
     // (starts with the next step), 2 running; the rows' ranges; the most cuboids each
@@ -415,7 +415,7 @@ struct sqd_core {
     unsigned long long split_fanout = 1;
     std::vector<std::uint32_t> st_subs, dyn_subs, dyn_initial;
     std::vector<double> box_init;                  // host copy of the compile-time box (uploaded per job)
-    unsigned long long range_init[3] = {0, 1, 1};  // host copy of the full initial range (and start flag)
+    unsigned long long range_init[2] = {0, 1};     // host copy of the full initial range
     // profiling: events around each launch, resolved at the next stream sync
     struct Pending { int kind; hipEvent_t a, b; };
     bool profiling = false;
@@ -435,8 +435,9 @@ enum : int { KIND_HULL_FINALIZE = 100, KIND_FINAL_NOSTATIC, KIND_INIT_HULL, KIND
 
 // A static level's kernels are named after how the core decides it: the
 // binary32 prefilter with binary64 for the undecided children, the binary64
-// group test, or the plain binary64 pass.
-sqd_kernel_stat make_stat(int kind, const sqd_settings& settings) {
+// group test (the last of the n_static levels, and where it is asked for), or
+// child by child in binary64.
+sqd_kernel_stat make_stat(int kind, const sqd_settings& settings, int n_static) {
     sqd_kernel_stat s{};
     static const char* modes[] = {"NONFINAL", "FINAL", "SPLIT", "INIT"};
     if(kind < 64) {
@@ -445,8 +446,8 @@ sqd_kernel_stat make_stat(int kind, const sqd_settings& settings) {
         const char* kernel = "dynamic_level";
         if(s.mode <= 1)
             kernel = ((settings.fp32_prefilter >> s.level) & 1u) ? "static_level_fp32"
-                   : ((settings.group_levels >> s.level) & 1u)  ? "static_level_group64"
-                                                                 : "static_level";
+                   : ((settings.group_levels >> s.level) & 1u) || s.level == n_static - 1 ? "static_level_group64"
+                                                                                          : "static_level";
         std::snprintf(s.name, sizeof s.name, "%s<%s,%d>", kernel, modes[s.mode], s.level);
     } else {
         s.mode = -1;
@@ -492,7 +493,7 @@ void sync(sqd_core* c) {
         float ms = 0;
         hip_check(hipEventElapsedTime(&ms, p.a, p.b), "hipEventElapsedTime");
         auto it = c->stats.find(p.kind);
-        if(it == c->stats.end()) it = c->stats.emplace(p.kind, make_stat(p.kind, c->settings)).first;
+        if(it == c->stats.end()) it = c->stats.emplace(p.kind, make_stat(p.kind, c->settings, c->ks->NSTAT)).first;
         it->second.launches += 1;
         it->second.milliseconds += ms;
     }
@@ -916,9 +917,9 @@ void report_progress(sqd_core* c, unsigned long long rounds, bool done, int stat
     c->progress_fn(c->progress_user, &pr);
 }
 
-// Captures the launches and copies that `enqueue` makes on the core's stream
-// into an executable HIP graph (kernels and one device-to-host copy; nothing
-// that needs a memset node).
+// Captures the launches that `enqueue` makes on the core's stream
+// into an executable HIP graph (kernels only, the state goes to the host from the
+// last one; nothing that needs a memset node).
 template<typename F> hipGraphExec_t capture_graph(sqd_core* c, F&& enqueue) {
     std::lock_guard<std::mutex> lock(g_capture_mutex);
     hipGraph_t g = nullptr;
@@ -1127,11 +1128,12 @@ void prove_steps(sqd_core* c) {
 // Proves the initial ranges [first[j], last[j]) of n jobs, leaving each job's
 // final state in h_state[j].  A core of one job runs one grid row; a batch core
 // always runs all its rows (the jobs beyond n get empty ranges and do no work),
-// so that its captured graphs fit every call.  One host round trip per round:
-// the round's size is decided on the device, the host only learns whether some
-// frontier is left.  From the second proof on a core (the first one fills the
-// launch statistics), the rounds are replayed as captured graphs unless
-// profiling is on.  Progress reports (single jobs only) follow job 0.
+// so that one layout of launches fits every call.  One host round trip per round:
+// the round's size is decided on the device, the host only learns what its lists
+// hold.  A proof runs in steps (prove_steps); with profiling, a critical sink or
+// progress reports it runs whole rounds, which are replayed as captured graphs from
+// the second proof on a core unless profiling is on.  Progress reports (single jobs
+// only) follow job 0.
 void prove_jobs(sqd_core* c, unsigned n, const uint32_t* first, const uint32_t* last, double* seconds,
                 bool progress_reports) {
     const uint32_t all = c->dyn_initial.empty() ? 1u : static_cast<uint32_t>(c->dyn_initial[0]);
@@ -1314,7 +1316,7 @@ void configure_core(sqd_core* c, int device, const sqd_program* program, const s
     c->crit.lay(lay, c->N, s.critical_capacity, false, false);
     c->scratch.lay(lay, c->N, std::max<unsigned long long>(kmax, 1024), true, false);
     lay.take(c->d_hull, static_cast<std::size_t>(kmax) * c->N * 4);
-    lay.take(c->d_range, 3);   // first, last, start flag
+    lay.take(c->d_range, 2);   // first, last
     if(c->fp32) {
         c->undec_cap = undec_cap;
         lay.take(c->d_undec, static_cast<std::size_t>(undec_cap));
@@ -1366,7 +1368,6 @@ void upload_job_constants(sqd_core* c) {
     const auto& prog = c->program->prog;
     c->range_init[0] = 0ull;
     c->range_init[1] = c->dyn_initial.empty() ? 1ull : c->dyn_initial[0];
-    c->range_init[2] = 1ull;
     c->box_init.assign(prog.box_lb.begin(), prog.box_lb.end());
     c->box_init.insert(c->box_init.end(), prog.box_ub.begin(), prog.box_ub.end());
     const std::size_t n_consts = 2 * static_cast<std::size_t>(std::max(1, c->ks->NC));
