@@ -56,7 +56,8 @@ typedef struct sqd_settings {
     uint32_t generation_count;     /* generations of dynamic splits (reference default 8) */
     uint32_t dequeue_buffer_size;  /* dynamic cuboids per round; default chosen per program */
     uint64_t frontier_capacity;    /* cuboids the device frontier can hold; default 1<<23 */
-    uint64_t level_bytes;          /* bytes per level buffer; default 1<<30 */
+    uint64_t level_bytes;          /* bytes per level buffer, which bounds a round's cuboids (the
+                                      lists take a little more); default 1<<30 */
     uint64_t critical_capacity;    /* criticals the device list holds (default 1<<20; at least the
                                       last static level's subdivisions): more fail a call unless a
                                       critical sink receives them (sqd_core_set_critical_sink) */
@@ -264,8 +265,9 @@ int sqd_core_acos_fallbacks(sqd_core* core, uint64_t* n);
 
 /* With sqd_settings.fp32_prefilter set: the static-level children of the last
  * computing call (sqd_prove, sqd_nonfinal, sqd_final) that the binary32 pass
- * evaluated, and those it decided (pruned) without binary64.  No counterpart in
- * the reference. */
+ * evaluated, and those it decided (pruned) without binary64 (none in a host-driven
+ * pass over boxes outside the program's compile-time box, which is all binary64).
+ * No counterpart in the reference. */
 int sqd_core_fp32_stats(sqd_core* core, uint64_t* checked, uint64_t* decided);
 
 /* Binary32-versus-binary64 overestimation per constraint: over n boxes (SoA,

@@ -26,7 +26,7 @@
 //   deps(list, f)            calls f(a) for each bound index a in update list `list`
 //   rows_violated<L>(lb, ub, C)   constraint rows of static level L
 //   all_satisfied(lb, ub, C)      every remaining constraint possibly holds
-//   level_waves(L), prop_fast(L)  per-level register budget (0: the default) and propagation form
+//   prop_fast(L)             per-level propagation form
 #pragma once
 #include <type_traits>
 #include "interval.hpp"
@@ -46,20 +46,18 @@ constexpr int kBlock = 256;
 #else
 #define SQD_LEVEL_ATTR
 #endif
-// The binary64 static level kernels take their program's budget for the level
-// (P::level_waves(L)) or else 3 waves, unless SQD_LEVEL_WAVES_PER_EU is set.  3
-// waves allow 168 VGPRs: Four's level 1 (180 and 2 waves left to the compiler) 305
-// -> 242 us for 3.3 M children (48 bytes of scratch), the levels that needed less
-// unchanged; 4 waves made More2's level 1 214 -> 262 us.
-template<class P, int L>
-constexpr int static_level_waves() {
-    return SQD_LEVEL_WAVES_PER_EU > 0 ? SQD_LEVEL_WAVES_PER_EU : (P::level_waves(L) > 0 ? P::level_waves(L) : 3);
-}
-
+// Waves per SIMD that the static kernels keep at least, in binary64 child by child:
+// 3 waves allow 168 VGPRs.  Four's level 1 (180 and 2 waves left to the compiler; 20
+// of them spilled now) 305 -> 242 us for 3.3 M children, the levels that needed less
+// unchanged; 4 waves made More2's level 1 214 -> 262 us.  On a last level, which is
+// the pass over the children binary32 left undecided, 3 and 4 waves are the same
+// (One, Two and Three, prefiltered levels of one and of eight jobs, within 0.5%).
+constexpr int kLevelWaves = SQD_LEVEL_WAVES_PER_EU > 0 ? SQD_LEVEL_WAVES_PER_EU : 3;
 // The kernel with the group test holds both the test and the per-child decision;
-// left to the compiler More2's takes 262 VGPRs and one wave per SIMD.  3 waves:
-// More2's level 733 -> 481 us, the others within 2%; 4 waves spill (More1 42 ->
-// 174 ms).
+// left to the compiler More2's takes 262 VGPRs and one wave per SIMD.  3 waves
+// (More2's spills 107 VGPRs, More1's 70, Four's 36, Three's 33, Two's and One's
+// none): More2's level 733 -> 481 us, the others within 2%; at 4 waves More1's took
+// 174 ms instead of 42.
 constexpr int kGroupWaves = 3;
 
 enum Mode : int { NONFINAL = 0, FINAL = 1, SPLIT = 2, INIT = 3 };
@@ -717,7 +715,7 @@ __device__ __forceinline__ void static_decide(const LevelArgs& args, const Input
 // F32 = true: the children listed in args.undec (by k_static_prefilter, those
 // binary32 left undecided) are decided in binary64, exactly as above.
 template<class P, int MODE, int L, bool F32>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(static_level_waves<P, L>())))
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kLevelWaves)))
 void k_static_level(LevelArgs job0) {
     const LevelArgs args = job_args(job0);
     constexpr int SUBS = P::st_subs(L);
@@ -1226,7 +1224,10 @@ __global__ __launch_bounds__(kBlock) void k_hull_finalize(BoxList items, const u
 // A round up to its dynamic split without static variables, one block per job:
 // the round's cuboids are taken from the frontier; each is its own only leaf and
 // hull and goes to `spl` with depth + 1 or, at the last generation, to `fin` and
-// to the criticals.  (Three kernels before, 4 to 5 us each for a few cuboids.)
+// to the criticals.  Three kernels did this before, 4 to 5 us each for a few cuboids;
+// one block is the faster one in large rounds too: ec1 at 12 generations, with rounds
+// of 8,192 cuboids, 542 us a proof against 730, and 32 jobs of it at 10 generations
+// 853 against 1,026.
 template<class P>
 __global__ __launch_bounds__(kBlock) void k_round_nostatic(BoxList stack, RoundWords* round, unsigned long long k_max,
                                                            unsigned long long fanout, BoxList fin, BoxList spl,

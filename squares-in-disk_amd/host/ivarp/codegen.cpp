@@ -558,25 +558,10 @@ std::string generate(const flat::Program& p, const std::string& key) {
     table("dyn_subs", dyn, [](const flat::FSplit& s) { return static_cast<int>(s.subs); });
     table("st_arg", sta, [](const flat::FSplit& s) { return s.arg; });
     table("st_subs", sta, [](const flat::FSplit& s) { return static_cast<int>(s.subs); });
-    // Register budget of the per-child binary64 level kernels (k_static_level) as
-    // resident waves per SIMD (0: the kernels' default).  On a last level that is
-    // the pass over the children binary32 left undecided; the values were measured
-    // on whole levels decided child by child: One's and Two's level 1 at 4 (128
-    // VGPRs, a few spilled; 3 was slower), Three's level 1 at 4 (274 against 292
-    // us), More1's level 1 at 3 (264 against 301 ms at the compiler's 176 VGPRs),
-    // Four's level 2 at 3 (3.46 against 3.92 ms) and More2's level 2 at 3 (19.8 ms;
-    // 4 spilled 426 VGPRs and took 38.7 ms).
-    int waves_l1 = 0, waves_l2 = 0;
-    if(key == "one" || key == "two" || key == "three") waves_l1 = 4;
-    if(key == "more1") waves_l1 = 3;
-    if(key == "four" || key == "more2") waves_l2 = 3;
-    o << "    static constexpr int level_waves(int l) { return l == 1 ? " << waves_l1 << " : l == 2 ? " << waves_l2
-      << " : 0; }\n";
     // Whether the static levels' propagation applies the initial bounds inline
     // before it builds its queue (same results; fewer instructions, more
-    // registers).  Measured per kernel: faster for every statement's dominant
-    // level but Four's level 2 (193 instead of 171 VGPRs: 2 waves per SIMD
-    // instead of 3, 4.72 against 4.37 ms per proof).
+    // registers).  Faster everywhere but on Four's level 2, whose kernels spill
+    // more with it (683 against 691 us a proof, 3.40 against 3.49 ms for seven).
     int slow_prop_level = -1;
     if(key == "four") slow_prop_level = 2;
     o << "    static constexpr bool prop_fast(int l) { return l != " << slow_prop_level << "; }\n";
