@@ -38,8 +38,9 @@ checked against the published ones.  The line printed carries
   ratio_decomposition
               the batched leg's ratio split into its causes, on One and on
               Four, every configuration through the same service shape
-              (`--workers` x `--batch-jobs`): plain binary64 in batches (no
-              group test, no prefilter), the binary64 group test in batches,
+              (`--workers` x `--batch-jobs`): plain binary64 in batches (the
+              group test on the last level alone, no prefilter), the binary64
+              group test on every level in batches,
               and the FP32-first service (autotuned); ratios to the plain
               batched rate
   legs        the other configurations of the metric, each with its counts
@@ -55,9 +56,9 @@ checked against the published ones.  The line printed carries
                                   service with autotuned settings, the FP32
                                   decided fraction and width ratios
                 more1_fp32_first  >=5 Subcontainers, s_n <= sigma, y_3 <= 0
-                                  (1,056,154,896 cuboids) with HIP-graph
-                                  rounds and the frontier in HBM, plain
-                                  binary64 and FP32-first (autotuned)
+                                  (1,056,154,896 cuboids) with the
+                                  frontier in HBM, plain binary64 and
+                                  FP32-first (autotuned)
   job_stream  proof jobs over all 11 statements (statement uniform, a
               contiguous 1/2^k slice of the first variable's initial
               subdivisions, k uniform in 0..6, seeded) through a service with a
@@ -84,6 +85,11 @@ sys.path.insert(0, str(ROOT / "squares-in-disk_amd"))
 METRIC = "cuboids/sec + p50/p99 proof-job latency, FP32-first batched vs plain FP64, 1 GPU"
 FP64_PEAK_TFLOPS = 78.6          # MI355X binary64 vector peak
 SIMDS, CLOCK_HZ, VALU_CYCLES = 1024, 2.4e9, 4   # MI355X: 256 CUs x 4 SIMDs; a wave64 VALU op holds a SIMD 4 cycles
+# what the rooflines' operations count (a kernel with the group test makes fewer evaluations)
+FLOPS_BASIS = ("one evaluation per cuboid; a group test decides up to 32 cuboids with one, so on levels that have "
+               "it achieved and frac are the work done, not the operations made")
+# the launches that the kernel times come from
+PROFILED_LAUNCHES = "whole rounds, empty final and split levels among them, which timed proofs do not launch"
 PUBLISHED = {                    # (cuboids, leaves) from the reference's prover output
     "top1": (128, 128), "top2": (168, 168), "one": (2869888, 2858678), "two": (7181696, 7069587),
     "three": (3549856, 3440786), "four": (37245328, 35026303), "five": (3392, 3188), "six": (14848, 13928),
@@ -128,7 +134,7 @@ def parse():
     ap.add_argument("--no-legs", action="store_true", help="skip the Four and More1 legs")
     ap.add_argument("--legs", default="four,more1", help="which of the Four and More1 legs to run")
     ap.add_argument("--no-graphs", action="store_true",
-                    help="cores launch every round's kernels directly instead of replaying HIP graphs "
+                    help="cores launch whole rounds directly instead of replaying them as HIP graphs "
                          "(the same kernels; for counter collection)")
     ap.add_argument("--no-decomposition", action="store_true", help="skip the batched-ratio decomposition")
     ap.add_argument("--leg-proofs", type=int, default=64, help="batched Four proofs per configuration")
@@ -479,7 +485,7 @@ def leg_roofline(stat, phases, fp32=False):
     frac = a64 / FP64_PEAK_TFLOPS + a32 / FP32_PEAK_TFLOPS       # share of the launch the ops need at peak
     peak = (a64 + a32) / frac if frac else FP64_PEAK_TFLOPS
     return {"bound": "valu", "achieved": a64 + a32, "peak": peak, "unit": "TFLOP/s", "frac": frac,
-            "traffic": None, "kernel": stat["name"], "mean_launch_ms": mean_ms,
+            "traffic": None, "kernel": stat["name"], "mean_launch_ms": mean_ms, "flops_basis": FLOPS_BASIS,
             "children_per_launch": children, "flops_per_launch": f64 + f32,
             "binary64_ops_per_child": ph[0] / ph[1], "binary32_ops_per_child": ph[2] / ph[1] if fp32 else 0.0,
             "achieved_binary64": a64, "achieved_binary32": a32}
@@ -491,16 +497,17 @@ def lemma_leg(sqd, key, plain_steps, sample_cuboids, workers, batch_jobs, proofs
     expected = PUBLISHED[key]
     out = {"lemma": key, "cuboids_per_proof": expected[0], "leaves_per_proof": expected[1],
            "reference_published_seconds": PUBLISHED_SECONDS.get(key)}
-    # plain binary64, reference split policy, HIP-graph rounds, frontier in HBM
+    # plain binary64, reference split policy, frontier in HBM
     with sqd.Core(prog, settings=sqd.default_settings(generation_count=8)) as core:
         core.prove()
         stats = profiled_proof(sqd, core, expected)
-        core.prove()                                          # captures the round graphs
+        core.prove()
         out["plain_fp64"] = timed_proofs(core, expected, plain_steps)
     dom = dominant(stats)
+    out["kernel_ms_launches"] = PROFILED_LAUNCHES
     out["plain_fp64"]["kernel_ms_per_proof"] = {s["name"]: s["milliseconds"] for s in
                                                 sorted(stats, key=lambda s: -s["milliseconds"])[:4]}
-    # FP32-first on a core of one job (autotuned), HIP-graph rounds
+    # FP32-first on a core of one job (autotuned)
     best, tune = sqd.autotune(prog, base=sqd.default_settings(), fp32_first=True)
     with sqd.Core(prog, settings=best) as core:
         core.prove()
@@ -734,7 +741,7 @@ def main():
             "bound": "valu", "achieved": achieved, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
             "frac": achieved / FP64_PEAK_TFLOPS, "traffic": traffic,
             "kernel": dom["name"], "mean_launch_ms": mean_ms, "launches_per_proof": launches_per_proof,
-            "flops_per_launch": flops_per_launch,
+            "flops_basis": FLOPS_BASIS, "flops_per_launch": flops_per_launch,
             "cuboids_per_launch": cuboids_per_proof / launches_per_proof,
             "flops_per_cuboid": flops_per_proof / cuboids_per_proof if cuboids_per_proof else None,
             "valu_issue_bound_ms": issue_ms,
@@ -757,6 +764,7 @@ def main():
                    "split_policy": "reference", "generations": 8, "cuboids_per_proof": expected[0],
                    "leaves_per_proof": expected[1]},
         "latency_ms": {"p50": percentile(lat, 0.5) * 1e3, "p99": percentile(lat, 0.99) * 1e3},
+        "warmup_kernel_launches": PROFILED_LAUNCHES,
         "warmup_kernel_ms_per_step": {s["name"]: s["milliseconds"] / max(1, a.warmup) for s in
                                       sorted(warm, key=lambda s: -s["milliseconds"])},
         "roofline": roofline,
