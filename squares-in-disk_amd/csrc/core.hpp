@@ -940,10 +940,11 @@ __global__ __launch_bounds__(kBlock) SQD_LEVEL_ATTR void k_static_prefilter(Leve
 // per-child path runs on full waves.  Nothing leaves the kernel but what survives,
 // and a level is one launch.
 //
-// Bound by VALU issue and latency (2 to 3 waves per SIMD).  Against one evaluation
-// per child: One's level 1 (2.8 M children) 75 -> 20 us, Three's (3.3 M) 276 -> 23
-// us, Four's level 2 (33.7 M) 3.43 -> 0.21 ms, More2's (115 M) 14.2 -> 0.48 ms,
-// More1's level 1 (1.01 G over 160 rounds) 258 -> 42 ms.
+// Bound by VALU issue and latency (3 waves per SIMD).  Against one evaluation per
+// child: One's level 1 (2.8 M children, 95 K tests) 75 -> 17 us, Three's (3.3 M, 104
+// K) 276 -> 23 us, Four's level 2 (33.7 M, 2.1 M) 3.43 -> 0.21 ms, More2's (115 M,
+// 7.2 M) 14.2 -> 0.48 ms, More1's level 1 (1.01 G over 160 rounds, 129 M tests and 83
+// M children decided by themselves) 258 -> 42 ms.
 template<class P, int MODE, int L>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kGroupWaves)))
 void k_static_grouped(LevelArgs job0) {
@@ -977,7 +978,6 @@ void k_static_grouped(LevelArgs job0) {
     const unsigned split = static_cast<unsigned>(cpl / part);    // parts of a group (at most 4)
     const unsigned per = 64u / static_cast<unsigned>(part);   // listed groups that make 64 children
     unsigned nq = 0, nl = 0;                                     // wave-uniform list sizes
-    unsigned untested = 0;                                       // trips of groups to leave untested
     unsigned long long next = static_cast<unsigned long long>(blockIdx.x) * (kBlock / 64) + wib;
     unsigned long long c_cub = 0, c_leaf = 0, c_crit = 0;
     for(;;) {
@@ -1019,9 +1019,7 @@ void k_static_grouped(LevelArgs job0) {
         }
         bool keep = valid;
         const bool whole = len != part;
-        if(whole && untested > 0) {
-            --untested;   // straight to the parts
-        } else if(valid) {
+        if(valid) {
             const int i = static_cast<int>(w % SUBS);
             double lb[N], ub[N];
             load_box<P>(args.in, w / SUBS, lb, ub);
@@ -1037,9 +1035,6 @@ void k_static_grouped(LevelArgs job0) {
         const unsigned long long m = __ballot(keep);
         const unsigned at = static_cast<unsigned>(__popcll(m & below)), n = static_cast<unsigned>(__popcll(m));
         if(whole) {
-            // a first test that leaves more than three quarters of the groups costs
-            // more than it saves: the next groups go to their parts untested
-            if(untested == 0 && 4u * n > 3u * static_cast<unsigned>(__popcll(__ballot(valid)))) untested = 16;
             if(keep)
                 for(unsigned k = 0; k < split; ++k) parts[nq + split * at + k] = w + k * static_cast<unsigned>(part);
             nq += split * n;

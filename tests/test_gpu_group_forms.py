@@ -1,8 +1,7 @@
 """The group tests where groups really form: with one or three blocks per launch the
 children of a level take many trips, so that the first test runs, its groups are
-split, listed, left untested and decided in ragged waves.  Decisions, hulls and
-criticals are the oracle's bit for bit (it decides every child by itself), so no
-tolerance is involved."""
+split, listed and decided in ragged waves.  Decisions, hulls and criticals are the
+oracle's bit for bit (it decides every child by itself), so no tolerance is involved."""
 import numpy as np
 import pytest
 
