@@ -1264,9 +1264,8 @@ void configure_core(sqd_core* c, int device, const sqd_program* program, const s
     // of a level's children and two waves more.  That slack and the counters come on
     // top of level_bytes (for One 250 KB and 8 KB per job), so that a round and a
     // host-driven call take as many cuboids as with dense lists.  Lists that the
-    // slack would lengthen by more than a quarter stay dense: their levels append at
-    // most 128 waves on one counter, 1.5 us (1,152 with a group test before the
-    // last level, 14 us).
+    // slack would more than double stay dense: their levels append at most 32 waves
+    // on one counter, 0.4 us (288 with a group test before the last level, 3.5 us).
     unsigned n_lists = 0;
     for(int mode : {dev::NONFINAL, dev::FINAL})
         for(std::size_t L = 0; L + 1 < c->st_subs.size() && n_lists < sizeof(SegIndex); ++L)
@@ -1280,7 +1279,7 @@ void configure_core(sqd_core* c, int device, const sqd_program* program, const s
     const unsigned before_last = used >> 1;
     const unsigned long long slack = 64ull * dev::kSegs * ((s.group_levels & before_last) ? dev::kSegs + 2 : 2);
     const unsigned long long room = lvl_cap;   // entries the rounds may fill
-    if(segments && n_lists > 0 && lvl_cap + slack < (1ull << 32) && lvl_cap >= 4 * slack) {
+    if(segments && n_lists > 0 && lvl_cap + slack < (1ull << 32) && lvl_cap >= slack) {
         c->segs.n_lists = n_lists;
         lvl_cap += slack;
     }

@@ -56,7 +56,7 @@ def _pieces(program_text, m):
 
 
 # ec3: an entry of a level list has 60 bytes, and the first static level 8 children
-@pytest.mark.parametrize("limit", [200, 1200])                # dense and segmented lists
+@pytest.mark.parametrize("limit", [200, 256, 1200])           # dense lists, and segmented ones from 256 on
 def test_host_calls_take_as_many_boxes_as_level_bytes_allow(program_text, limit):
     lb, ub = _pieces(program_text, limit // 4)
     o = pyoracle.Oracle(program_text("ec3"))
@@ -75,11 +75,13 @@ def test_host_calls_take_as_many_boxes_as_level_bytes_allow(program_text, limit)
             assert e.value.code == -4
 
 
-@pytest.mark.parametrize("n,kw", [(1200, {}), (9216, dict(group_levels=0xFFFFFFFF, prefilter_group=8)),
-                                  (9216, dict(group_levels=0xFFFFFFFF, prefilter_group=8, grid_blocks=3))])
+@pytest.mark.parametrize("n,kw", [(256, {}), (1200, {}), (9216, dict(group_levels=0xFFFFFFFF, prefilter_group=8)),
+                                  (9216, dict(group_levels=0xFFFFFFFF, prefilter_group=8, grid_blocks=3)),
+                                  (2304, dict(group_levels=0xFFFFFFFF, prefilter_group=2, grid_blocks=1))])
 def test_segments_filled_to_their_bound(program_text, n, kw):
-    # the largest round of the smallest lists kept in segments (longer ones where the
-    # first level has a group test), all children of the first level surviving
+    # the largest round of lists kept in segments, the smallest ones among them (2,048
+    # entries; 18,432 where the first level has a group test), all children of the
+    # first level surviving
     lb, ub = _pieces(program_text, n // 4)
     ohl, ohu, ohas, oc = pyoracle.Oracle(program_text("ec3")).nonfinal(lb, ub)
     assert oc["num_cuboids"] == n * (8 + 1024)
