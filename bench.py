@@ -120,7 +120,7 @@ def parse():
     ap.add_argument("--batched-settings", default=None, metavar="K=V,...",
                     help="fixed settings of the batched leg (e.g. fp32_prefilter=2,prefilter_group=8) instead of "
                          "autotuning them; for reproducible profiles")
-    ap.add_argument("--traffic", default=str(ROOT / "profiles" / "traffic_static_level_one_subcontainer.txt"),
+    ap.add_argument("--traffic", default=str(ROOT / "profiles" / "traffic_static_level_group64_one_subcontainer.txt"),
                     help="HBM traffic summary (FETCH_SIZE/WRITE_SIZE per dispatch) to attach to the roofline")
     ap.add_argument("--workers", type=int, default=4, help="batches in flight in the batched legs")
     ap.add_argument("--batch-jobs", type=int, default=32, help="proofs per batch (one grid row each)")
